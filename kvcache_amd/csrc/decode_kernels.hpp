@@ -560,18 +560,21 @@ __global__ __launch_bounds__(WPB * kWave) void split_kernel(const int* __restric
         // blocks the chunk touches (0 for an empty chunk); the planner keeps this
         // within kMaxChunkBlocks, the min() only guards the LDS staging
         const int nblk = min(j1 > j0 ? (j1 - 1) / p.block - b0 + 1 : 0, kMaxChunkBlocks);
-        // The block ids are read through a descriptor: on the planned path the
-        // descriptor spans table_all (table_len ints), so any plan reads inside it;
-        // otherwise it spans this chunk's nblk entries.
+        // The block ids are read through a descriptor that ends with this chunk's nblk
+        // entries (a lane past them reads 0 and touches no memory) and, on the planned
+        // path, inside table_all (table_len ints), so any plan reads inside it.  A
+        // device-length launch carries no table length: there the chunk's own end is the
+        // only bound, and a table may end where its allocation does.
         // (a short sequence of a self-planned launch: its own entries)
         constexpr bool WHOLE_TABLE = PLANNED && !LEAD;
         const int first = tab_start + (PLANNED ? 0 : b0);
         const __amdgpu_buffer_rsrc_t trs =
-            WHOLE_TABLE ? tile_rsrc(p.table_all, p.table_len * 4) : tile_rsrc(p.table_all + first, nblk * 4);
+            WHOLE_TABLE ? tile_rsrc(p.table_all, min(p.table_len, first + nblk) * 4)
+                        : tile_rsrc(p.table_all + first, nblk * 4);
         const int tb = WHOLE_TABLE ? first * 4 : 0;  // byte offset of the chunk's first entry
         if constexpr (UNIFORM) {
-            // unconditional: lanes past the chunk's blocks read a neighbour's id or 0 and
-            // are never selected by the readlane below
+            // unconditional: lanes past the chunk's blocks read 0 and are never selected by
+            // the readlane below (but for loads past the chunk's rows, of zero size)
             tbl = (int)__builtin_amdgcn_raw_buffer_load_b32(trs, tb + lane * 4, 0, 0);
         } else {
             for (int b = threadIdx.x; b < nblk; b += WPB * kWave)

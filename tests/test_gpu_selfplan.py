@@ -20,6 +20,8 @@ from kvcache_amd import KVC_F16, KVC_F32, ops
 from kvcache_amd import workloads as W
 from kvcache_amd._native import KVC_ERR_ARG, KvcError
 from kvcache_amd.device import DeviceBuffer
+from kvcache_amd.engine import BlockAllocator
+from kvcache_amd.workloads import build_tables
 
 from _helpers import as_np, dev, host, normal, paged_layout, say, tol, tuning
 
@@ -356,3 +358,37 @@ def test_short_sequences_while_planning(orc, case):
         np.testing.assert_array_equal(a, b)
         np.testing.assert_array_equal(a, contig)
         assert np.all(a[lens == 0] == 0)
+
+
+@pytest.mark.parametrize("n,causal", [(1, False), (5, False), (3, True)])
+def test_block_table_at_the_end_of_its_allocation(orc, n, causal):
+    # device-length launches carry no table length: every table read has to stay within
+    # the blocks of the chunk it is for (each lane of a wave reads one entry of a chunk
+    # that may have fewer than 64), also where the table's allocation ends with it
+    say(f"table at the end of its allocation n={n} causal={causal}")
+    Hq = Hkv = 8
+    D, B, base = 64, 16, 4000
+    lens = np.array([4001 - 300 * i for i in range(n)], np.int32) if not causal else np.array([base + n], np.int32)
+    alloc = BlockAllocator(int(sum((int(x) + B - 1) // B for x in lens)))
+    alloc.shuffle(3)
+    table, off = build_tables(lens, B, alloc)
+    kp, vp = (normal((alloc.total_blocks, Hkv, B, D), 40 + i, np.float16) for i in range(2))
+    q = normal((n, Hq, D), 42, np.float16)
+    room = 2 << 20  # a whole allocation unit: the table's last entry is its last four bytes
+    buf = DeviceBuffer(room)
+    full = np.zeros(room // 4, np.int32)
+    full[-len(table):] = table
+    buf.upload(full)
+    tab = buf.ptr + room - 4 * len(table)
+    out = DeviceBuffer(q.nbytes)
+    if causal:
+        pos = DeviceBuffer.from_numpy(np.array([base], np.int32))
+        ops.qkcuda_paged_causal_attn(dev(q), out, dev(kp), dev(vp), tab, pos, n, Hq, Hkv, D, B, 0.125)
+        ref = orc.batched_paged(q, kp, vp, np.tile(table, n), np.arange(n + 1, dtype=np.int32) * len(table),
+                                base + 1 + np.arange(n, dtype=np.int32), Hkv, B, 0.125)
+    else:
+        ops.launch_batched_paged(dev(q), dev(kp), dev(vp), tab, DeviceBuffer.from_numpy(off),
+                                 DeviceBuffer.from_numpy(lens), out, n, Hq, D, B, 0, 0.125, Hkv=Hkv, dtype=KVC_F16)
+        ref = orc.batched_paged(q, kp, vp, table, off, lens, Hkv, B, 0.125)
+    got = host(out, np.float16, q.shape).astype(np.float64)
+    assert np.abs(got - ref).max() <= 2e-3
