@@ -104,6 +104,7 @@ struct Plan {
     bool chunk_blocks_ok = true;  // the per-lane path stages at most 4096 block ids per chunk
     size_t acc_bytes = 0, ml_bytes = 0, ws_bytes = 0;
     size_t n_ctr = 0;  // arrival counters
+    int qtile = 0;     // prompt attention: queries per workgroup
 };
 
 inline int ilog2_exact(int x) {  // log2 of a power of two, else -1
@@ -585,7 +586,7 @@ int guarded(F&& f) {
 
 inline hipStream_t S(kvc_stream_t s) { return static_cast<hipStream_t>(s); }
 
-// ---- prompt attention on the matrix cores: 16 queries of one head per unit ----
+// ---- prompt attention on the matrix cores (prompt_mfma.hpp) ----
 bool causal_tile_path(int Nq, int Hq, int Hkv, int D, int BLOCK, int dtype) {
     if (tuning().mfma == 0 || dtype != KVC_F16 || (D != 64 && D != 128) || BLOCK <= 0 || BLOCK % 16 ||
         (BLOCK & (BLOCK - 1)))
@@ -594,26 +595,44 @@ bool causal_tile_path(int Nq, int Hq, int Hkv, int D, int BLOCK, int dtype) {
     return (long long)Nq * Hq * D * 2 < (1LL << 31);  // the q descriptor spans all queries
 }
 
-// Key chunks: enough units (query tiles x heads x chunks) to fill the CUs about
-// twice, chunks of at least 512 tokens and at most 1024 blocks.
+// Queries per workgroup, from how many workgroups there would be.  head_dim 64: 32 (key
+// streams of their own, two workgroups per CU) until tiles of 64 give two per CU as well
+// (14 heads: 2048 queries 22.3 us at 32, 22.8 at 64; 4096 queries 64.9 and 58.2 us).
+// head_dim 128: the largest tile that still gives about 160 workgroups (32 heads: 200
+// queries 8.0 us at 32, 9.8 at 64; 450 queries 14.9, 13.0, 16.0 us at 32, 64, 128; 2048
+// queries 94.7, 76.4, 59.8 us).
+int prompt_qtile(int Nq, int Hq, int D) {
+    auto wgs = [&](int t) { return (long long)((Nq + t - 1) / t) * Hq; };
+    if (D == 64) return wgs(64) >= 512 ? 64 : 32;
+    return wgs(128) >= 160 ? 128 : wgs(64) >= 160 ? 64 : 32;
+}
+
+// Chunks a tile's keys may be split into (32-query tiles only: few workgroups, long
+// prefixes): up to one workgroup per CU, of at least prompt_min_chunk keys (one query of
+// 14 heads behind 20000 keys: 13.6 us with up to 256 workgroups, 15.5 with 128, 16.9 with
+// 512; 20 queries of 32 heads, D 128, behind 5900: 22.2 us in chunks of 1024, 26 of 1536).
+int prompt_max_chunks(int Nq, int Hq) {
+    const long long wgs = (long long)((Nq + 31) / 32) * Hq;
+    return (int)std::min(64LL, std::max(1LL, 256 / wgs));
+}
+int prompt_min_chunk(int D) { return D == 64 ? 512 : 1024; }
+
 Plan plan_causal_tile(int base, int Nq, int Hq, int Hkv, int D, int BLOCK) {
     Plan pl;
     pl.mfma = true;
     pl.G = Hq / Hkv;
     pl.nsub = 1;
     pl.mode = kCausalTile;
+    pl.wpb = 8;
+    pl.qtile = prompt_qtile(Nq, Hq, D);
     const long long lmax = std::max(1LL, (long long)base + Nq);
-    const long long tiles = (long long)((Nq + 15) / 16) * Hq;
-    const long long want = std::max(1LL, (512 + tiles - 1) / std::max(tiles, 1LL));
-    long long ch = std::max<long long>(512, (lmax + want - 1) / want);
-    long long p2 = 1;
-    while (p2 < ch) p2 <<= 1;
-    ch = std::min<long long>(p2, (long long)kMfmaMaxChunkBlocksHost * BLOCK);
-    ch = (ch + BLOCK - 1) / BLOCK * BLOCK;
+    long long nch = 1;
+    if (pl.qtile == 32 && lmax >= kPromptSplitMin)
+        nch = std::min<long long>(prompt_max_chunks(Nq, Hq), std::max(1LL, lmax / prompt_min_chunk(D)));
+    const long long al = std::max(BLOCK, 256);
+    const long long ch = std::min<long long>((lmax + nch * al - 1) / (nch * al) * al, INT_MAX);
     pl.chunk = (int)ch;
     pl.max_chunks = (int)((lmax + ch - 1) / ch);
-    const int t = tuning().waves_per_block;
-    pl.wpb = (t == 4 || t == 8) ? t : (tiles * pl.max_chunks >= 512 ? 4 : 8);
     size_workspace(pl, Nq, Hq, Hkv, D);
     return pl;
 }
@@ -640,6 +659,7 @@ int run_causal_tile(const void* q, void* out, const void* k, const void* v, cons
     L.dtype = KVC_F16; L.D = D; L.G = pl.G; L.mode = kCausalTile; L.wpb = pl.wpb; L.batch = tuning().batch;
     L.need_merge = pl.max_chunks > 1;
     L.mfma = true;
+    L.qtile = pl.qtile;
     return launch_decode(L, st);
 }
 
@@ -830,6 +850,19 @@ int run_self_planned(const void* q, const void* k, const void* v, const int* tab
     if (cap > 0) upper = std::min(upper, (long long)ps.hks * N * ((long long)cap / std::max(ps.min_chunk, 1) + 2));
     if (tuning().self_grid > 0) upper = std::min(upper, (long long)tuning().self_grid);
     L.units = (int)std::min<long long>(std::max(upper, 1LL), INT_MAX);
+    // prompt queries at a device position: prompt_stream_kernel, whose tiles share their
+    // keys' loads (14q/2kv, 96 queries behind 1500 keys 14.2 -> 10.9 us, 400 behind 4000
+    // 87 -> 21 us; 8 heads, one query behind 1500 10.9 -> 9.9 us).  Up to 7 queries of
+    // grouped heads stay with the decode units, which read each key once for the group: at
+    // 60000 keys and one query 18 us against 25 (at 4000, 15.4 against 9.5)
+    if (!contig && !cur_len && (N >= 8 || !ps.mfma) && causal_tile_path(N, Hq, Hkv, D, BLOCK, dtype) &&
+        (long long)((N + 31) / 32) * Hq <= recs) {
+        L.mode = kCausalTile;
+        L.mfma = true;
+        L.qtile = 32;
+        p.max_chunks = std::min(prompt_max_chunks(N, Hq), kSelfRecordsPerHeadHost);
+        p.sp_min_chunk = prompt_min_chunk(D);
+    }
     return launch_decode(L, st);
 }
 

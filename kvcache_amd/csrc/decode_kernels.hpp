@@ -939,6 +939,7 @@ __global__ __launch_bounds__(kMergeThreads) void merge_kernel(DecodeParams p) {
 }
 
 #include "gqa_mfma.hpp"
+#include "prompt_mfma.hpp"
 
 // Dynamic LDS that caps workgroups per CU (tuning "wg_per_cu"), from the
 // kernel's static LDS (queried once per kernel).
@@ -1066,7 +1067,11 @@ int launch_gqa_mode(DecodeLaunch L, dim3 grid, hipStream_t st) {
         case kContiguous:     L.lds_pad = lds_pad(gqa_mfma_kernel<D, kContiguous, WPB>, L.wg_per_cu); hipLaunchKernelGGL((gqa_mfma_kernel<D, kContiguous, WPB>), grid, block, L.lds_pad, st, L.p.work, L.p.work_ints, L.p); break;
         case kPagedUniform:   L.lds_pad = lds_pad(gqa_mfma_kernel<D, kPagedUniform, WPB>, L.wg_per_cu); hipLaunchKernelGGL((gqa_mfma_kernel<D, kPagedUniform, WPB>), grid, block, L.lds_pad, st, L.p.work, L.p.work_ints, L.p); break;
         case kPlannedUniform: L.lds_pad = lds_pad(gqa_mfma_kernel<D, kPlannedUniform, WPB>, L.wg_per_cu); hipLaunchKernelGGL((gqa_mfma_kernel<D, kPlannedUniform, WPB>), grid, block, L.lds_pad, st, L.p.work, L.p.work_ints, L.p); break;
-        case kCausalTile:     hipLaunchKernelGGL((gqa_mfma_kernel<D, kCausalTile, WPB>), grid, block, 0, st, L.p.work, L.p.work_ints, L.p); break;
+        case kCausalTile:
+            if (L.qtile == 128) hipLaunchKernelGGL((prompt_kernel<D, 4, 8>), grid, dim3(8 * kWave), 0, st, L.p);
+            else if (L.qtile == 64) hipLaunchKernelGGL((prompt_kernel<D, 2, 8>), grid, dim3(8 * kWave), 0, st, L.p);
+            else hipLaunchKernelGGL((prompt_stream_kernel<D, 1>), grid, dim3(8 * kWave), 0, st, L.p);
+            break;
         case kSelfPlanned:
             L.lds_pad = lds_pad(gqa_mfma_kernel<D, kSelfPlanned, WPB>, L.wg_per_cu);
             grid = self_grid(gqa_mfma_kernel<D, kSelfPlanned, WPB>, block.x, L.lds_pad, grid, L.p);
@@ -1105,7 +1110,7 @@ int launch_decode_d(const DecodeLaunch& L, hipStream_t st) {
     const bool planned = L.mode == kPlannedUniform || L.mode == kPlannedPerLane || L.mode == kSelfPlanned ||
                          L.mode == kSelfContig;
     const long long units = planned ? (long long)L.units
-                          : L.mode == kCausalTile ? (long long)L.p.max_chunks * ((L.p.N + 15) / 16) * L.p.Hq
+                          : L.mode == kCausalTile ? (long long)L.p.max_chunks * ((L.p.N + L.qtile - 1) / L.qtile) * L.p.Hq
                                                   : (long long)L.p.max_chunks * L.p.N * L.p.Hkv * L.p.nsub;
     if (units <= 0) return KVC_OK;
     if (units > (long long)INT_MAX) return set_error(KVC_ERR_ARG, "decode grid too large");

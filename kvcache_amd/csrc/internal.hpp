@@ -19,7 +19,7 @@ int hip_check(hipError_t e, const char* what);
 // ---------------------------------------------------------------------------
 // kPlanned*: the grid is a host-built work list (kvc_decode_plan) instead of a
 // (chunk, sequence, head) decomposition; otherwise as kPaged*.
-// kCausalTile (matrix-core kernel only): prompt attention, a unit is 16 consecutive
+// kCausalTile (prompt_mfma.hpp): prompt attention, a workgroup is qtile consecutive
 // queries of one query head over one chunk of keys of the shared block table.
 // kSelfPlanned: lengths in device memory; every workgroup of a persistent grid
 // derives the host planner's units itself (selfplan.hpp) and serves ranks
@@ -109,6 +109,11 @@ int* device_error_word(hipStream_t st, bool may_alloc);
 bool take_device_error_code(int code);
 int device_error_status(int code);
 
+// Prompt attention with fewer keys than this is never split over workgroups: up to here
+// one workgroup's key streams take about as long as a split's partials and merge (14
+// heads, D 64: 100 queries behind 2000 tokens 12.2 us whole, 13.5 us in chunks of 512).
+constexpr int kPromptSplitMin = 3072;
+
 // Arrival counters.  Atomics that land on one 128-byte line serialise (about 10 ns
 // each on MI355X, whether or not they hit the same address), so counters that are
 // hot together must not share a line: counter i goes to line i mod L, word i / L
@@ -147,6 +152,7 @@ struct DecodeLaunch {
     int wpb;     // waves per workgroup (4 or 8); one workgroup per unit
     int batch;   // wave-loads per double-buffered batch (2, 4 or 8; used for G <= 2)
     int units;   // planned launches: number of work-list units (the grid); else 0
+    int qtile;   // kCausalTile: queries per workgroup (32: prompt_stream_kernel; 64 or 128: prompt_kernel)
     bool need_merge;
     bool mfma;   // grouped-query matrix-core kernel (fp16, head_dim 64/128, G = group <= 16)
     unsigned lds_pad;  // dynamic LDS bytes reserved per workgroup (occupancy cap)

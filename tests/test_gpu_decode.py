@@ -460,6 +460,36 @@ def test_paged_causal_attn(orc, dtype, Hq, Hkv, base, n):
         assert np.abs(got - host(alt, nt, q.shape).astype(np.float64)).max() <= 2e-3
 
 
+# the tiles of the prompt kernels: 32 queries (few workgroups), 64 (D 64 from 512 workgroups
+# of them, D 128 from 160), 128 (D 128 from 160); keys in sets of 128 or streams of 256, the
+# split of few queries behind at least 3072 keys, blocks of 16 to 64 tokens
+@pytest.mark.parametrize("D,Hq,Hkv,B,base,n", [
+    (64, 14, 2, 16, 0, 31), (64, 14, 2, 16, 1, 33), (64, 3, 3, 32, 255, 65), (64, 5, 1, 64, 63, 129),
+    (64, 128, 4, 16, 0, 255), (64, 128, 2, 32, 17, 225),           # 64-query tiles
+    (64, 2, 1, 16, 3071, 1), (64, 2, 1, 16, 3070, 1), (64, 14, 2, 16, 6000, 33),  # split and not
+    (128, 8, 2, 16, 127, 32), (128, 8, 2, 64, 4100, 5),
+    (128, 64, 2, 16, 0, 150), (128, 64, 4, 32, 100, 129),          # 64-query tiles
+    (128, 64, 2, 16, 0, 257), (128, 160, 4, 32, 129, 128)])         # 128-query tiles
+@pytest.mark.parametrize("device_pos", [False, True])
+def test_prompt_tiles(orc, D, Hq, Hkv, B, base, n, device_pos):
+    say(f"prompt tiles D={D} Hq={Hq} Hkv={Hkv} B={B} base={base} n={n} device_pos={device_pos}")
+    nb = (base + n + B - 1) // B
+    table = np.random.default_rng(base + n).permutation(nb + 3)[:nb].astype(np.int32)
+    kp, vp = normal((nb + 3, Hkv, B, D), 210, np.float16), normal((nb + 3, Hkv, B, D), 211, np.float16)
+    q = normal((n, Hq, D), 212, np.float16)
+    scale = -0.11  # (a negative scale negates q)
+    out = DeviceBuffer(q.nbytes)
+    if device_pos:
+        ops.qkcuda_paged_causal_attn(dev(q), out, dev(kp), dev(vp), dev(table), dev(np.array([base], np.int32)), n, Hq,
+                                     Hkv, D, B, scale)
+    else:
+        ops.qk_paged_causal_attn(dev(q), out, dev(kp), dev(vp), dev(table), base, n, Hq, Hkv, D, B, scale)
+    got = host(out, np.float16, q.shape).astype(np.float64)
+    want = orc.paged_causal(q, kp, vp, table, base, Hkv, B, scale, nthreads=8)
+    # the path's fp16 bar (tol): the probabilities' and the output's fp16 rounding
+    assert np.abs(got - want).max() <= tol(KVC_F16)
+
+
 def test_prefill_flow_write_then_causal_attn(orc):
     """The model path's prefill (qwen_serve.cu:106-108): write the P prompt rows of
     K/V through the sequence's table, then causal attention over them."""
