@@ -151,9 +151,10 @@ Plan plan_batched_mfma(int N, int Hq, int Hkv, int D, int BLOCK, int cap, int sp
     if (paged && ch % BLOCK) ch = (ch + BLOCK - 1) / BLOCK * BLOCK;
     pl.chunk = (int)std::min<long long>(ch, 1 << 24);
     pl.max_chunks = std::max(1, (std::max(cap, 0) + pl.chunk - 1) / pl.chunk);
-    // 4 waves per unit once there are enough units to fill the CUs, else 8
+    // 4 waves per unit once there are enough units to fill the CUs (head_dim 128: always,
+    // as plan_shape), else 8
     const int t = tuning().waves_per_block;
-    pl.wpb = (t == 4 || t == 8) ? t : ((long long)pl.max_chunks * N * Hkv >= 256 ? 4 : 8);
+    pl.wpb = (t == 4 || t == 8) ? t : (D == 128 || (long long)pl.max_chunks * N * Hkv >= 256 ? 4 : 8);
     pl.mode = paged ? kPagedUniform : kContiguous;
     pl.chunk_blocks_ok = !paged || pl.chunk / BLOCK <= kMfmaMaxChunkBlocksHost;
     size_workspace(pl, N, Hq, Hkv, D);
@@ -391,30 +392,43 @@ constexpr int kPlanIntsInline = 64;   // grouped-query units: header + up to 56 
 
 struct PlanShape {
     int G, nsub, hks, tpw, wpb, min_chunk, max_chunk, slots, entry_ints;
+    int min_chunk_long = 0;  // mfma: min_chunk for batches with long sequences (plan_min_chunk)
     int target_cap = INT_MAX;  // largest automatic chunk target (tokens)
     bool uniform, mfma;
 };
 
-PlanShape plan_shape(int Hq, int Hkv, int D, int BLOCK, int dtype) {
+// N: sequences of the launch (waves per unit only; the units do not depend on it).
+PlanShape plan_shape(int Hq, int Hkv, int D, int BLOCK, int dtype, int N = 0) {
     PlanShape ps{};
     const int group = Hq / Hkv;
     if (mfma_path(group, D, dtype, BLOCK, true)) {
-        // all heads of the group per unit; 8 waves; at least two 32-token tiles per
-        // wave; about 0.7 units per CU: each unit streams ~1000 tokens, which keeps
-        // the chunks of long sequences few (their fused merge is the tail)
+        // all heads of the group per unit; at least two 32-token tiles per wave
         ps.mfma = true;
         ps.uniform = true;
         ps.G = group;
         ps.nsub = 1;
         ps.hks = Hkv;
         ps.tpw = 32;
+        // head_dim 128: 4 waves (8 spill 41-125 registers and leave no CU a second unit:
+        // 200 sequences of 32..4096 tokens, 32q/8kv, planned 209 -> 131 us, 16 sequences
+        // 28.3 -> 21.9).  head_dim 64: 8, and 4 once the units fill the chip several times
+        // (units of 64 lengths 14.8 us at 8 waves, 18.5 at 4; 500 x 2 19.8 and 15.9)
         const int t = tuning().waves_per_block;
-        ps.wpb = (t == 4 || t == 8) ? t : 8;
-        // a split costs the chunk tail a store, an arrival and a merge: below ~1024
-        // tokens a sequence stays in one unit
-        ps.min_chunk = ((tuning().mfma_min_chunk + BLOCK - 1) / BLOCK) * BLOCK;
+        ps.wpb = (t == 4 || t == 8) ? t : (D == 128 || (long long)N * Hkv >= 768 ? 4 : 8);
+        // a split costs the chunk tail a store, an arrival and a merge: sequences stay whole
+        // up to 1.5 chunks of at least min_chunk_long tokens, an eighth of the longest
+        // sequence between 512 (64 sequences of 128..4096 tokens 14.8 -> 13.6 us) and 1024
+        // (4 of 8192..32768: 15.3 us, 17.8 in chunks of 704), or min_chunk_long once whole
+        // sequences fill the CUs (60 sequences x 8 KV heads, D 128: 23.8 us, 27.0 in chunks
+        // of at least 512; 128 x 4, D 64: 15.1 and 16.1)
+        auto blocks_up = [&](int x) { return (x + BLOCK - 1) / BLOCK * BLOCK; };
+        ps.min_chunk = blocks_up(std::min(tuning().mfma_min_chunk, 512));
+        ps.min_chunk_long = blocks_up(tuning().mfma_min_chunk);
         ps.max_chunk = kMfmaMaxChunkBlocksHost * BLOCK;
-        ps.slots = 176;
+        // units to aim for: one per CU for head_dim 64; for 128 about two, whose shorter
+        // chunks balance the rounds of a large batch (200 sequences, device lengths: 172
+        // us aiming at 176 units, 160 at 256, 148 at 512)
+        ps.slots = D == 128 ? 512 : 256;
         // the unit's first block ids travel in its entry: the kernel reads entry and
         // ids in one round instead of entry, then table
         ps.entry_ints = kPlanIntsInline;
@@ -457,14 +471,27 @@ inline int plan_key(bool split, long long len, int T, bool split_first) {
 // chunks 0..nc-2 of every head, then the last chunk of every head).
 // The chunk target (tokens) of a plan: `target`, or automatically enough units to
 // fill the machine's slots about once, at least min_chunk, a multiple of BLOCK.
+// Least automatic or requested chunk for a batch of N sequences whose longest has lmax
+// tokens (the kernel's own planner applies the same rule).
+int plan_min_chunk(const PlanShape& ps, int N, int lmax, int BLOCK) {
+    if (!ps.mfma) return ps.min_chunk;
+    if ((long long)N * ps.hks >= kPlanFullUnits) return std::max(ps.min_chunk, ps.min_chunk_long);
+    const int eighth = (int)std::min<long long>(((long long)lmax / 8 + BLOCK - 1) / BLOCK * BLOCK, ps.min_chunk_long);
+    return std::max(ps.min_chunk, eighth);
+}
+
 int plan_chunk_target(const int* lens, int N, const PlanShape& ps, int BLOCK, int target) {
     long long total = 0;
-    for (int i = 0; i < N; ++i) total += std::max(lens[i], 1);
+    int lmax = 0;
+    for (int i = 0; i < N; ++i) {
+        total += std::max(lens[i], 1);
+        lmax = std::max(lmax, lens[i]);
+    }
     total *= ps.hks;
     if (target <= 0)
         target = (int)std::min<long long>(std::min<long long>((total + ps.slots - 1) / ps.slots, ps.target_cap),
                                           INT_MAX / 2);
-    int T = std::max(target, ps.min_chunk);
+    int T = std::max(target, plan_min_chunk(ps, N, lmax, BLOCK));
     T = (T + BLOCK - 1) / BLOCK * BLOCK;
     return std::min(T, ps.max_chunk);
 }
@@ -673,7 +700,7 @@ int run_planned(const void* q, const void* k_new, const void* v_new, const int* 
         if (BLOCK <= 0 || !table_all || table_len <= 0 || !work || n_units < 0 || n_records < 0)
             return set_error(KVC_ERR_ARG, "planned decode needs BLOCK > 0, a block table and a work list");
         if (!std::isfinite(scale)) return set_error(KVC_ERR_ARG, "scale must be finite");
-        const PlanShape ps = plan_shape(Hq, Hkv, D, BLOCK, dtype);
+        const PlanShape ps = plan_shape(Hq, Hkv, D, BLOCK, dtype, N);
         DecodeLaunch L{};
         DecodeParams& p = L.p;
         p.q = q; p.k = k_pool; p.v = v_pool; p.out = out;
@@ -785,7 +812,7 @@ int run_self_planned(const void* q, const void* k, const void* v, const int* tab
     if (contig) BLOCK = kSelfContigBlock;
     if (!contig && !table_all) return set_error(KVC_ERR_ARG, "null block table");
     if (!std::isfinite(scale)) return set_error(KVC_ERR_ARG, "scale must be finite");
-    const PlanShape ps = plan_shape(Hq, Hkv, D, BLOCK, dtype);
+    const PlanShape ps = plan_shape(Hq, Hkv, D, BLOCK, dtype, N);
     const long long bound = cap;  // the record budget follows the caller's stated bound
     const long long recs = self_plan_records(N, Hq, Hkv, D, BLOCK, dtype, bound);
     const size_t need = self_plan_workspace(N, Hq, Hkv, D, BLOCK, dtype, bound);
@@ -815,6 +842,7 @@ int run_self_planned(const void* q, const void* k, const void* v, const int* tab
     p.n_records = (int)recs;
     p.lpb_shift = ilog2_exact(BLOCK / ps.tpw);  // uniform paging (self_plan_ok)
     p.sp_slots = ps.slots; p.sp_min_chunk = ps.min_chunk; p.sp_max_chunk = ps.max_chunk;
+    p.sp_min_long = ps.min_chunk_long;
     p.sp_target_cap = ps.target_cap; p.sp_nc_max = ps.mfma ? kMfmaMaxFusedChunks : 0;
     p.sp_records = self_plan_budget(ps, bound);
     if (!contig && cur_len && tab_off && tuning().self_prefetch_kib > 0) {

@@ -70,8 +70,12 @@ __global__ __launch_bounds__(WPB * kWave) void gqa_mfma_kernel(const int* __rest
     constexpr int kMainBytes = 2 * WPB * kTileBytes;   // per wave: V tile, then K tile
     __shared__ __attribute__((aligned(16))) char s_buf[kMainBytes];
     __shared__ int s_tab[PAGED ? kMfmaMaxChunkBlocks : 1];
-    __shared__ float s_w[kMfmaMaxHeads][kMaxFusedChunks];
-    __shared__ float s_L[kMfmaMaxHeads];
+    // the fused merge's chunk weights and sums, over the tiles (whose partials have been
+    // read by then): with LDS of their own the self-planned kernels (D 64 with 8 waves, D
+    // 128 with 4) came to 82.8 KB, one workgroup per CU instead of two
+    static_assert((kMfmaMaxHeads * kMaxFusedChunks + kMfmaMaxHeads) * 4 <= kMainBytes, "weights fit the tiles");
+    float(*s_w)[kMaxFusedChunks] = reinterpret_cast<float(*)[kMaxFusedChunks]>(s_buf);
+    float* s_L = reinterpret_cast<float*>(s_buf) + kMfmaMaxHeads * kMaxFusedChunks;
     __shared__ int s_last;
     __shared__ std::conditional_t<SELF, SelfPlanLds<kSelfMaxNMfma, WPB>, char> s_plan;
 

@@ -77,6 +77,7 @@ struct DecodeParams {
     // queries whose first position lives in device memory, that position (query s
     // then attends to *dev_base + s + 1 keys; causal must be 1)
     int sp_slots, sp_min_chunk, sp_max_chunk, sp_target_cap;
+    int sp_min_long;          // matrix cores: sp_min_chunk of batches with long sequences (plan_min_chunk), else 0
     int sp_nc_max;            // chunks per sequence the merge can combine (0: any)
     int sp_records;           // partial records per (sequence, head) in the workspace
     int sp_pf_blocks;         // blocks of every sequence read ahead while the plan is made (0: none)
@@ -108,6 +109,10 @@ enum DeviceError {
 int* device_error_word(hipStream_t st, bool may_alloc);
 bool take_device_error_code(int code);
 int device_error_status(int code);
+
+// Grouped-query decode: with this many (sequence, KV head) pairs, one per CU, sequences are
+// only split into long chunks (plan_min_chunk).
+constexpr int kPlanFullUnits = 256;
 
 // Prompt attention with fewer keys than this is never split over workgroups: up to here
 // one workgroup's key streams take about as long as a split's partials and merge (14

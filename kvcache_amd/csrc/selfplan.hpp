@@ -118,9 +118,15 @@ __device__ __forceinline__ void self_split(const DecodeParams& p, int L, int T, 
 
 // Order bucket of a run of units of `len` tokens each: chunks of split sequences
 // (4..7) above whole sequences (0..3), longer above shorter, in quarters of 3T/8
-// (kscale = 8 / 3T).  Buckets only order the units; chunks, records and counters do
-// not depend on them.
+// (kscale = 8 / 3T).  HALVES (matrix cores): the whole sequences' edges are 3T/4, 3T/8 and
+// 3T/16, as T is far above most lengths of a large batch there.  Buckets only order the
+// units; chunks, records and counters do not depend on them.
+template <bool HALVES>
 __device__ __forceinline__ int self_bucket(bool split, int len, float kscale) {
+    if constexpr (HALVES) {
+        const float x = (float)len * kscale;
+        return split ? 4 + min(3, (int)x) : x >= 2.f ? 3 : x >= 1.f ? 2 : x >= 0.5f ? 1 : 0;
+    }
     return (split ? 4 : 0) + min(3, (int)((float)len * kscale));
 }
 
@@ -216,7 +222,13 @@ __device__ SelfPlan self_plan_setup(const int* lens, int n_seq, const DecodePara
         else if (pmax <= 0xFFFFFFFFull) c = ceil_div_u32((unsigned)prod, (unsigned)p.sp_slots);
         else c = ceil_div_u64((long long)prod, p.sp_slots);
         long long T = min(c, (long long)p.sp_target_cap);
-        T = max(T, (long long)p.sp_min_chunk);
+        long long least = p.sp_min_chunk;
+        if constexpr (!Lds::kLead) {  // matrix cores: plan_min_chunk's rule
+            const long long eighth = (long long)N * hks >= kPlanFullUnits ? (long long)p.sp_min_long
+                                                                        : (((long long)lall >> 3) + B - 1) >> bsh << bsh;
+            least = max(least, min(eighth, (long long)p.sp_min_long));
+        }
+        T = max(T, least);
         T = (T + B - 1) >> bsh << bsh;
         T = min(T, (long long)M);
         // ... raised to the record budget (and the 64-chunk merge of the matrix-core
@@ -256,8 +268,8 @@ __device__ SelfPlan self_plan_setup(const int* lens, int n_seq, const DecodePara
             self_split(p, L, Ti, bsh, nc, chunk);
             over |= nc > kSelfMaxChunks || L > p.cap;
             nc = min(nc, kSelfMaxChunks);
-            const int ka = self_bucket(nc > 1, chunk, kscale);
-            const int kb = self_bucket(nc > 1, nc > 1 ? L - (nc - 1) * chunk : L, kscale);
+            const int ka = self_bucket<!Lds::kLead>(nc > 1, chunk, kscale);
+            const int kb = self_bucket<!Lds::kLead>(nc > 1, nc > 1 ? L - (nc - 1) * chunk : L, kscale);
             S.cut[i] = nc | ((chunk >> bsh) << 16);
             S.bk[i] = ka | (kb << 4);
             const int ca = nc > 1 ? hks * (nc - 1) : 0;

@@ -392,3 +392,31 @@ def test_block_table_at_the_end_of_its_allocation(orc, n, causal):
         ref = orc.batched_paged(q, kp, vp, table, off, lens, Hkv, B, 0.125)
     got = host(out, np.float16, q.shape).astype(np.float64)
     assert np.abs(got - ref).max() <= 2e-3
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,n", [(64, 14, 2, 3), (64, 28, 4, 70), (64, 32, 8, 96), (128, 8, 2, 5),
+                                        (128, 32, 8, 33)])
+def test_grouped_units_host_and_device_plans(orc, D, Hq, Hkv, n):
+    # the grouped-query units' rules on the batch: fewer (sequence, KV head) pairs than
+    # kPlanFullUnits (chunks from an eighth of the longest sequence), at least that many,
+    # and at least 768 (4 waves at D 64); device lengths and host plan agree bit for bit
+    say(f"grouped units D={D} Hq={Hq} Hkv={Hkv} n={n}")
+    rng = np.random.default_rng(n)
+    lens = rng.integers(1, 400, n).astype(np.int32)
+    lens[:3] = (4200, 1549, 900)
+    B = 16
+    nb = int(sum((int(x) + B - 1) // B for x in lens))
+    alloc = BlockAllocator(nb)
+    alloc.shuffle(n)
+    table, off = build_tables(lens, B, alloc)
+    kp, vp = (normal((nb, Hkv, B, D), 60 + i, np.float16) for i in range(2))
+    q = normal((n, Hq, D), 62, np.float16)
+    scale = float(1.0 / np.sqrt(D))
+    got = self_planned(q, kp, vp, table, off, lens, Hkv, B, KVC_F16)
+    work, nu, nr = ops.decode_plan(lens, Hq, Hkv, D, B, tab_off=off, table=table)
+    out = DeviceBuffer(q.nbytes)
+    ops.launch_batched_paged_planned(dev(q), dev(kp), dev(vp), dev(table), len(table), out, n, Hq, Hkv, D, B, scale,
+                                     dev(work), nu, nr)
+    np.testing.assert_array_equal(got, host(out, np.float16, q.shape))
+    ref = orc.batched_paged(q, kp, vp, table, off, lens, Hkv, B, scale, nthreads=8)
+    assert np.abs(got.astype(np.float64) - ref).max() <= tol(KVC_F16)
