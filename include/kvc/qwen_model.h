@@ -11,8 +11,10 @@
 // RMSNorm + q/k/v projection + bias + rotary; the planned attention with the new
 // K/V written in the same launch; output projection + residual; RMSNorm + gate/up
 // projection + SwiGLU; down projection + residual; then final norm + lm_head +
-// argmax.  step_path 1 (and larger batches, and prompts) run one kernel per op with
-// rocBLAS linear layers; both round to fp16 at the same points.  With `graph` the
+// argmax.  Prompts and larger batches run RMSNorm and the fused linear layers of many rows
+// (kvc_block_qkv / swiglu / linear), with the prompts' K/V stored by the q/k/v kernel.
+// step_path 1 runs one kernel per op with rocBLAS linear layers; all round to fp16 at the
+// same points.  With `graph` the
 // fused step is captured once as a HIP graph whose kernels read the step's counts
 // (rows, attention units, partial records) from device memory; each step then
 // uploads its metadata into fixed places and replays the graph (the reference
@@ -78,6 +80,7 @@ struct QwenModel {
     void* rws = nullptr;  // fused kernels' workspace (zero between calls)
     size_t rws_bytes = 0;
     bool rows_ok = false;
+    bool block_ok = false;  // many rows: fused linear layers (kvc_block_*), else one kernel per op
     void* cws = nullptr;  // layer chain's workspace (its own: barrier counters persist between launches)
     size_t cws_bytes = 0;
     bool chain_ok = false;
@@ -139,6 +142,8 @@ struct QwenModel {
         kvc::check(kvc_host_alloc((void**)&h_tok, c.max_batch * 4), "pinned tokens");
         rows_ok = c.step_path == 0 && H % 32 == 0 && H <= 1024 && QD % 32 == 0 && I % 32 == 0 &&
                   c.vocab % 32 == 0 && c.head_dim % 32 == 0;
+        block_ok = c.step_path == 0 && H % 8 == 0 && QD % 8 == 0 && I % 8 == 0 &&
+                   (c.head_dim == 32 || c.head_dim == 64 || c.head_dim == 128);
         if (rows_ok) {
             rws_bytes = std::max({kvc_rows_workspace_size(H, QD), kvc_rows_workspace_size(H, I),
                                   kvc_rows_workspace_size(c.vocab, H)});
@@ -203,10 +208,27 @@ struct QwenModel {
     void* kl(int l) const { return kvm.k_layer(l); }
     void* vl(int l) const { return kvm.v_layer(l); }
 
-    // Rows [0, M) of x hold the layer input; attention is supplied by `attend(l)`.
+    // Rows [0, M) of x hold the layer input; attention is supplied by attend(l, written),
+    // `written` when the rows' K/V already lie in the pools (fused path with d_slots).
     template <typename Attend>
-    void layers(int M, const int* d_pos, int pos_base, Attend&& attend) {
+    void layers(int M, const int* d_pos, int pos_base, const int* d_slots, Attend&& attend) {
         const int H = c.hidden, QD = c.n_heads * c.head_dim, KD = c.n_kv_heads * c.head_dim, I = c.inter;
+        if (block_ok) {
+            for (int l = 0; l < c.layers; ++l) {
+                const Layer& w = L[l];
+                kvc::check(kvc_rmsnorm(nrm, x, w.ln1, M, H, c.eps, stream), "rmsnorm");
+                kvc::check(kvc_block_qkv(q, d_slots ? kl(l) : k, d_slots ? vl(l) : v, nrm, w.wq, w.bq, d_pos, pos_base,
+                                         d_slots, M, H, c.n_heads, c.n_kv_heads, c.head_dim, c.block_size, c.theta,
+                                         stream),
+                           "qkv + bias + rope");
+                attend(l, d_slots != nullptr);
+                kvc::check(kvc_block_linear(x, att, w.wo, M, H, QD, 1, stream), "o_proj + residual");
+                kvc::check(kvc_rmsnorm(nrm, x, w.ln2, M, H, c.eps, stream), "rmsnorm");
+                kvc::check(kvc_block_swiglu(gate, nrm, w.wg, M, I, H, stream), "gate/up + swiglu");
+                kvc::check(kvc_block_linear(x, gate, w.wd, M, H, I, 1, stream), "down_proj + residual");
+            }
+            return;
+        }
         for (int l = 0; l < c.layers; ++l) {
             const Layer& w = L[l];
             kvc::check(kvc_rmsnorm(nrm, x, w.ln1, M, H, c.eps, stream), "rmsnorm");
@@ -218,7 +240,7 @@ struct QwenModel {
             kvc::check(kvc_add_bias(v, w.bv, M, KD, stream), "v bias");
             kvc::check(kvc_rope(q, d_pos, pos_base, M, c.n_heads, c.head_dim, c.theta, stream), "rope q");
             kvc::check(kvc_rope(k, d_pos, pos_base, M, c.n_kv_heads, c.head_dim, c.theta, stream), "rope k");
-            attend(l);
+            attend(l, false);
             kvc::check(kvc_linear(o, att, w.wo, M, H, QD, KVC_F16, stream), "o_proj");
             kvc::check(kvc_add_residual(x, o, (size_t)M * H, stream), "residual");
             kvc::check(kvc_rmsnorm(nrm, x, w.ln2, M, H, c.eps, stream), "rmsnorm");
@@ -390,10 +412,11 @@ struct QwenModel {
         ensure_ws(kvc_decode_planned_workspace_size(c.n_heads, c.n_kv_heads, c.head_dim, c.block_size, KVC_F16, nr));
         kvc::check(kvc_embed_gather(x, embed, d_ids, R, c.hidden, c.vocab, stream), "embed");
         const float scale = 1.0f / __builtin_sqrtf((float)c.head_dim);
-        layers(R, d_pos, 0, [&](int l) {
-            kvc::check(kvc_write_kv_slots(k, v, kl(l), vl(l), d_slot, R, c.n_kv_heads, c.head_dim, c.block_size,
-                                          KVC_F16, stream),
-                       "prefill write_kv");
+        layers(R, d_pos, 0, d_slot, [&](int l, bool written) {
+            if (!written)
+                kvc::check(kvc_write_kv_slots(k, v, kl(l), vl(l), d_slot, R, c.n_kv_heads, c.head_dim, c.block_size,
+                                              KVC_F16, stream),
+                           "prefill write_kv");
             kvc::check(kvc_batched_paged_decode_planned(q, kl(l), vl(l), d_tabs, T, att, R, c.n_heads, c.n_kv_heads,
                                                         c.head_dim, c.block_size, scale, KVC_F16, d_work, nu, nr, ws,
                                                         ws_bytes, stream),
@@ -413,21 +436,26 @@ struct QwenModel {
         const int P = s.prompt_len;
         if (P <= 0 || P > c.max_rows) throw kvc::Error(KVC_ERR_ARG, "prefill: prompt length outside [1, max_rows]");
         const int nb = (int)s.block_table.size();
-        ensure_meta((size_t)P + nb);
+        // upload: [ids P | slot P | table nb]
+        ensure_meta(2 * (size_t)P + nb);
         kvc::check(kvc_stream_synchronize(stream), "meta reuse");
         std::memcpy(h_meta, tokens, P * 4);
-        std::memcpy(h_meta + P, s.block_table.data(), nb * 4);
-        kvc::check(kvc_step_upload(d_meta, h_meta, ((size_t)P + nb) * 4, stream), "prefill upload");
+        for (int r = 0; r < P; ++r)
+            h_meta[P + r] = s.block_table[r / c.block_size] * c.block_size + r % c.block_size;
+        std::memcpy(h_meta + 2 * P, s.block_table.data(), nb * 4);
+        kvc::check(kvc_step_upload(d_meta, h_meta, (2 * (size_t)P + nb) * 4, stream), "prefill upload");
         const int* d_ids = d_meta;
-        const int* d_table = d_meta + P;
+        const int* d_slot = d_meta + P;
+        const int* d_table = d_meta + 2 * P;
         ensure_ws(kvc_paged_causal_attn_workspace_size(0, P, c.n_heads, c.n_kv_heads, c.head_dim, c.block_size,
                                                        KVC_F16));
         kvc::check(kvc_embed_gather(x, embed, d_ids, P, c.hidden, c.vocab, stream), "embed");
         const float scale = 1.0f / __builtin_sqrtf((float)c.head_dim);
-        layers(P, nullptr, 0, [&](int l) {
-            kvc::check(kvc_write_kv(k, v, kl(l), vl(l), d_table, 0, P, c.n_kv_heads, c.head_dim, c.block_size,
-                                    KVC_F16, stream),
-                       "prefill write_kv");
+        layers(P, nullptr, 0, d_slot, [&](int l, bool written) {
+            if (!written)
+                kvc::check(kvc_write_kv(k, v, kl(l), vl(l), d_table, 0, P, c.n_kv_heads, c.head_dim, c.block_size,
+                                        KVC_F16, stream),
+                           "prefill write_kv");
             kvc::check(kvc_paged_causal_attn(q, att, kl(l), vl(l), d_table, 0, P, c.n_heads, c.n_kv_heads,
                                              c.head_dim, c.block_size, scale, KVC_F16, ws, ws_bytes, stream),
                        "prefill attention");
@@ -485,7 +513,7 @@ struct QwenModel {
         if (rows_ok && n <= kRowsMax) {
             rows_layers(n, d_pos, d_table, T, d_work, nu, nr);
         } else {
-            layers(n, d_pos, 0, [&](int l) {
+            layers(n, d_pos, 0, nullptr, [&](int l, bool) {
                 kvc::check(kvc_batched_paged_append_decode_planned(q, k, v, d_pos, kl(l), vl(l), d_table, T, att, n,
                                                                    c.n_heads, c.n_kv_heads, c.head_dim, c.block_size,
                                                                    scale, KVC_F16, d_work, nu, nr, ws, ws_bytes,

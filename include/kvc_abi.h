@@ -423,6 +423,23 @@ int kvc_rows_lm_head(float* logits, int* tokens, const void* x, const void* norm
                      kvc_stream_t stream);
 int kvc_rows_set_tuning(int splits, int groups_per_wg, int shape);
 
+/* ---- linear layers over many rows (prompts, steps of more than 32 sequences) ----
+ * Tiled matrix-core products with the operations after each layer fused in; rows
+ * already normalised (kvc_rmsnorm).  fp16 rows and weights ([out, in] row-major), fp32
+ * accumulation, results rounded to fp16 where the op-by-op path stores them.  Any M >= 0;
+ * N, K, I, H multiples of 8; pointers 16-byte aligned.
+ * kvc_block_linear: y[M,N] = x W^T, or y += x W^T when residual != 0; y must not be x.
+ * kvc_block_qkv: q|k|v = x [wq;wk;wv]^T + [bq;bk;bv], rotary embedding of q and k at
+ *   position pos[r] (pos NULL: pos_base + r); q [M, Hq*D]; k and v [M, Hkv*D], or, with
+ *   slots (slots[r] = phys*BLOCK + pos%BLOCK, negative: not written), straight into the
+ *   paged pools [num_blocks, Hkv, BLOCK, D] (kvc_write_kv_slots); D 32, 64 or 128.
+ * kvc_block_swiglu: act[M,I] = silu(x wg^T) * (x wu^T), w_gate_up = [wg; wu] as [2I, H]. */
+int kvc_block_linear(void* y, const void* x, const void* w, int M, int N, int K, int residual, kvc_stream_t stream);
+int kvc_block_qkv(void* q, void* k, void* v, const void* x, const void* w_qkv, const void* b_qkv, const int* pos,
+                  int pos_base, const int* slots, int M, int H, int Hq, int Hkv, int D, int BLOCK, float theta,
+                  kvc_stream_t stream);
+int kvc_block_swiglu(void* act, const void* x, const void* w_gate_up, int M, int I, int H, kvc_stream_t stream);
+
 /* The linear layers between two attention launches of a decode step as ONE launch:
  * the tail of layer l -- x += att W_o^T; act = silu(n W_g^T) * (n W_u^T) with
  * n = RMSNorm(x) * ln2; x += act W_d^T -- then the head of layer l + 1 -- q|k|v =

@@ -172,6 +172,9 @@ _SIGS = {
     "kvc_graph_launch": (i32, [vp, vp]),
     "kvc_graph_destroy": (i32, [vp]),
     "kvc_rows_set_tuning": (i32, [i32, i32, i32]),
+    "kvc_block_linear": (i32, [vp, vp, vp, i32, i32, i32, i32, vp]),
+    "kvc_block_qkv": (i32, [vp] * 7 + [i32, vp] + [i32] * 6 + [f32, vp]),
+    "kvc_block_swiglu": (i32, [vp, vp, vp, i32, i32, i32, vp]),
     "kvc_rows_chain_workspace_size": (sz, [i32, i32]),
     "kvc_rows_chain": (i32, [vp, vp, sz, vp]),
     "kvc_flash_decode": (i32, [vp, vp, vp, vp, i32, i32, i32, i32, f32, i32, i32, vp, sz, vp]),

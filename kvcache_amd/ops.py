@@ -262,6 +262,25 @@ def rows_lm_head(logits, tokens, x, w, M, V, H, *, norm_w=None, eps=1e-6, dev_ro
                                  wsb, stream))
 
 
+# ---- linear layers over many rows (fused matrix-core kernels) ------------------------
+def block_linear(y, x, w, M, N, K, *, residual=False, stream=None):
+    """y[M,N] = x w^T, or y += x w^T (residual)."""
+    check(lib().kvc_block_linear(_p(y), _p(x), _p(w), M, N, K, int(residual), stream))
+
+
+def block_qkv(q, k, v, x, w_qkv, b_qkv, M, H, Hq, Hkv, D, theta, *, pos=None, pos_base=0, slots=None, BLOCK=0,
+              stream=None):
+    """q|k|v = x [wq;wk;wv]^T + bias, rotary on q and k at pos[r] (or pos_base + r); with
+    slots, k and v are the paged pools."""
+    check(lib().kvc_block_qkv(_p(q), _p(k), _p(v), _p(x), _p(w_qkv), _p(b_qkv), _p(pos), pos_base, _p(slots), M, H, Hq,
+                              Hkv, D, BLOCK, theta, stream))
+
+
+def block_swiglu(act, x, w_gate_up, M, I, H, *, stream=None):
+    """act = silu(x wg^T) * (x wu^T), w_gate_up = [wg; wu]."""
+    check(lib().kvc_block_swiglu(_p(act), _p(x), _p(w_gate_up), M, I, H, stream))
+
+
 def rows_chain_workspace_size(H, I) -> int:
     return int(lib().kvc_rows_chain_workspace_size(H, I))
 

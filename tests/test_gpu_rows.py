@@ -424,3 +424,72 @@ def test_chain_other_shape_and_refusal():
         assert np.array_equal(host(acta, np.uint16, (M_, I)), host(actb, np.uint16, (M_, I)))
         for a, b, n in ((qa, qb, qd), (ka, kb, kd), (va, vb, kd)):
             assert np.array_equal(host(a, np.uint16, (M_, n)), host(b, np.uint16, (M_, n)))
+
+
+# ---- linear layers over many rows (tiled kernels) ---------------------------------------
+# rows and columns around the 64- and 128-wide tiles, K around the 64-wide blocks and the K
+# groups (two; four from K 2048 on with few tiles), tiles of 128 from 200 of them
+@pytest.mark.parametrize("M_,N,K", [(1, 8, 8), (33, 72, 104), (64, 64, 128), (65, 136, 896), (129, 896, 4864),
+                                    (1700, 2048, 72), (1700, 2040, 2056)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_block_linear(M_, N, K, residual):
+    say(f"block linear M={M_} N={N} K={K} residual={residual}")
+    x = normal((M_, K), 500, np.float16)
+    w = (normal((N, K), 501) / np.sqrt(K)).astype(np.float16)
+    y0 = normal((M_, N), 502, np.float16)
+    y = dev(y0)
+    ops.block_linear(y, dev(x), dev(w), M_, N, K, residual=residual)
+    ref = _r16(M.linear(x.astype(np.float32), w))
+    close(host(y, np.float16, (M_, N)), y0.astype(np.float64) + ref if residual else ref)
+
+
+@pytest.mark.parametrize("M_,Hq,Hkv,D,H", [(1, 14, 2, 64, 896), (70, 14, 2, 64, 896), (40, 4, 2, 32, 104),
+                                           (130, 4, 1, 128, 256), (2900, 14, 2, 64, 64)])
+@pytest.mark.parametrize("slots", [False, True])
+def test_block_qkv(M_, Hq, Hkv, D, H, slots):
+    say(f"block qkv M={M_} Hq={Hq} Hkv={Hkv} D={D} H={H} slots={slots}")
+    theta, B = 1e6, 16
+    QD, KD = Hq * D, Hkv * D
+    x = normal((M_, H), 510, np.float16)
+    w = (normal((QD + 2 * KD, H), 511) / np.sqrt(H)).astype(np.float16)
+    b = (0.5 * normal((QD + 2 * KD,), 512)).astype(np.float16)
+    rng = np.random.default_rng(513)
+    pos = rng.integers(0, 4000, M_).astype(np.int32)
+    q = DeviceBuffer(M_ * QD * 2)
+    y = _r16(_r16(M.linear(x.astype(np.float32), w)) + b.astype(np.float32))
+    if slots:  # rows at random places of the pools, every seventh row not written; positions 5 + row
+        nb = M_ // B + 2
+        slot = rng.permutation(nb * B)[:M_].astype(np.int32)
+        slot[::7] = -1
+        pool0 = normal((nb, Hkv, B, D), 514, np.float16)
+        kp, vp = dev(pool0), dev(pool0)
+        ops.block_qkv(q, kp, vp, dev(x), dev(w), dev(b), M_, H, Hq, Hkv, D, theta, pos_base=5, slots=dev(slot), BLOCK=B)
+        pos = 5 + np.arange(M_, dtype=np.int32)
+    else:
+        kp, vp = DeviceBuffer(M_ * KD * 2), DeviceBuffer(M_ * KD * 2)
+        ops.block_qkv(q, kp, vp, dev(x), dev(w), dev(b), M_, H, Hq, Hkv, D, theta, pos=dev(pos))
+    rq = M.rope(y[:, :QD].reshape(M_, Hq, D), pos, D, theta).reshape(M_, QD)
+    rk = M.rope(y[:, QD:QD + KD].reshape(M_, Hkv, D), pos, D, theta).reshape(M_, KD)
+    close(host(q, np.float16, (M_, QD)), rq)
+    if not slots:
+        close(host(kp, np.float16, (M_, KD)), rk)
+        close(host(vp, np.float16, (M_, KD)), y[:, QD + KD:])
+        return
+    for got, want in ((host(kp, np.float16, pool0.shape), rk), (host(vp, np.float16, pool0.shape), y[:, QD + KD:])):
+        rows = got.transpose(0, 2, 1, 3).reshape(nb * B, KD)  # [slot, Hkv * D]
+        old = pool0.transpose(0, 2, 1, 3).reshape(nb * B, KD)
+        used = slot >= 0
+        close(rows[slot[used]], want[used])
+        rest = np.setdiff1d(np.arange(nb * B), slot[used])
+        np.testing.assert_array_equal(rows[rest], old[rest])
+
+
+@pytest.mark.parametrize("M_,I,H", [(1, 8, 8), (65, 40, 136), (130, 4864, 896), (1700, 1032, 72)])
+def test_block_swiglu(M_, I, H):
+    say(f"block swiglu M={M_} I={I} H={H}")
+    x = normal((M_, H), 520, np.float16)
+    w = (normal((2 * I, H), 521) / np.sqrt(H)).astype(np.float16)
+    act = DeviceBuffer(M_ * I * 2)
+    ops.block_swiglu(act, dev(x), dev(w), M_, I, H)
+    g, u = _r16(M.linear(x.astype(np.float32), w[:I])), _r16(M.linear(x.astype(np.float32), w[I:]))
+    close(host(act, np.float16, (M_, I)), M.silu_mul(g, u))
