@@ -78,7 +78,7 @@ struct RowsParams {
     int q_cols, kv_cols, head_dim;
     const int* dev_rows;     // graph-safe launches: the step's row count in device memory (M is then a capacity)
     float* logits;           // logits: fp32 [M, N] or nullptr
-    float* best_v;           // logits: [groups][kRows] per-group row maxima
+    float* best_v;           // logits: [workgroups][kRows] row maxima of each workgroup's groups
     int* best_i;
 };
 
@@ -205,7 +205,7 @@ __device__ __forceinline__ void epilogue(const RowsParams& p, int M, int g, int 
         const auto r = rsrc(p.logits, p.logits ? M * p.N * 4 : 0);
         st_f<CP>(r, (mm * p.N + c0) * 4, v0);
         st_f<CP>(r, (mm * p.N + c1) * 4, v1);
-        if (m < M) {  // (no memory access inside)
+        if (ok && m < M) {  // (no memory access inside)
             better(bv, bi, v0, c0);
             better(bv, bi, v1, c1);
         }
@@ -485,19 +485,6 @@ __device__ __forceinline__ bool run_group(const Lane& ln, const RowsParams& p, i
         float bv = -FLT_MAX;
         int bi = INT_MAX;
         epilogue<EPI, CP>(p, M, ok ? g : g0, m, c, v[it][0], v[it][1], ok, e[it], bv, bi);
-        if constexpr (EPI == kEpiLogits) {
-            // the 16 column pairs of row m sit in 16 consecutive lanes
-#pragma unroll
-            for (int o = 1; o < 16; o <<= 1) {
-                const float ov = __shfl_xor(bv, o);
-                const int oi = __shfl_xor(bi, o);
-                better(bv, bi, ov, oi);
-            }
-            // one lane per row stores the group's candidate (rows >= M are never read)
-            const int o = ok && c == 0 ? (g * kRows + m) * 4 : kOob;
-            st_f<0>(rsrc(p.best_v, p.groups * kRows * 4), o, bv);
-            __builtin_amdgcn_raw_buffer_store_b32((unsigned)bi, rsrc(p.best_i, p.groups * kRows * 4), o, 0, 0);
-        }
     }
     return true;
 }
@@ -649,6 +636,15 @@ __global__ __launch_bounds__(WAVES * 64) void rows_kernel(RowsParams p) {
         }
     }
 
+    // logits: each thread's best output over this workgroup's groups (its row and lane
+    // column are the same in every group)
+    float bv[kItems];
+    int bi[kItems];
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) {
+        bv[it] = -FLT_MAX;
+        bi[it] = INT_MAX;
+    }
     // One column group: MFMAs over this wave's k range, sum over the waves, epilogue.
     // `ok` false (a group past the end) runs the same code with every store dropped.
     // Returns false when this workgroup is not the last of a split group (it is done).
@@ -744,22 +740,7 @@ __global__ __launch_bounds__(WAVES * 64) void rows_kernel(RowsParams p) {
 #pragma unroll
         for (int it = 0; it < kItems; ++it) {
             const int item = threadIdx.x + it * kThreads, m = item / 16, c = item % 16;
-            float bv = -FLT_MAX;
-            int bi = INT_MAX;
-            epilogue<EPI, 0>(p, M, ok ? g : g0, m, c, v[it][0], v[it][1], ok, e[it], bv, bi);
-            if constexpr (EPI == kEpiLogits) {
-                // the 16 column pairs of row m sit in 16 consecutive lanes
-#pragma unroll
-                for (int o = 1; o < 16; o <<= 1) {
-                    const float ov = __shfl_xor(bv, o);
-                    const int oi = __shfl_xor(bi, o);
-                    better(bv, bi, ov, oi);
-                }
-                // one lane per row stores the group's candidate (rows >= M are never read)
-                const int o = ok && c == 0 ? (g * kRows + m) * 4 : kOob;
-                st_f<0>(rsrc(p.best_v, p.groups * kRows * 4), o, bv);
-                __builtin_amdgcn_raw_buffer_store_b32((unsigned)bi, rsrc(p.best_i, p.groups * kRows * 4), o, 0, 0);
-            }
+            epilogue<EPI, 0>(p, M, ok ? g : g0, m, c, v[it][0], v[it][1], ok, e[it], bv[it], bi[it]);
         }
         return true;
     };
@@ -773,6 +754,24 @@ __global__ __launch_bounds__(WAVES * 64) void rows_kernel(RowsParams p) {
             run_group(b0, e0, j, true);
             load_b(b0, e0, g0 + j + 2, j + 2 < ng);
             run_group(b1, e1, j + 1, j + 1 < ng);
+        }
+    }
+    if constexpr (EPI == kEpiLogits) {
+        // one candidate per row and workgroup: the 16 column pairs of row m sit in 16
+        // consecutive lanes (rows >= M are never read)
+#pragma unroll
+        for (int it = 0; it < kItems; ++it) {
+            const int item = threadIdx.x + it * kThreads, m = item / 16, c = item % 16;
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) {
+                const float ov = __shfl_xor(bv[it], o);
+                const int oi = __shfl_xor(bi[it], o);
+                better(bv[it], bi[it], ov, oi);
+            }
+            if (c == 0) {
+                p.best_v[unit * kRows + m] = bv[it];
+                p.best_i[unit * kRows + m] = bi[it];
+            }
         }
     }
 }
@@ -937,7 +936,8 @@ __global__ __launch_bounds__(kChainWaves * 64) void chain_kernel(ChainParams cp)
     if constexpr (HEAD) chain_phase<kEpiQkv, true, false, MT, 1>(cp.ph[kPhQ], M, cp.units[kPhQ], wb, L, [] {});
 }
 
-// tokens[m] = the column of the largest candidate over the groups (first index on ties).
+// tokens[m] = the column of the largest candidate over the workgroups (first index on
+// ties): 475 per row at 151936 outputs (one per column group, 4748, took 12 to 16 us).
 constexpr int kArgThreads = 256;
 __global__ __launch_bounds__(kArgThreads) void group_argmax_kernel(const float* best_v, const int* best_i, int groups,
                                                                    int* tokens, const int* dev_rows) {
@@ -1214,7 +1214,7 @@ int kvc_rows_lm_head(float* logits, int* tokens, const void* x, const void* norm
                     : launch_rows<kEpiLogits, false>(p, one, (hipStream_t)st);
         if (rc) return rc;
         hipLaunchKernelGGL(group_argmax_kernel, dim3(M), dim3(kArgThreads), 0, (hipStream_t)st, p.best_v, p.best_i,
-                           groups, tokens, dev_rows);
+                           (groups + one.gpw - 1) / one.gpw, tokens, dev_rows);
         return hip_check(hipGetLastError(), "argmax launch");
     } catch (...) {
         return set_error(KVC_ERR_STATE, "unexpected exception");

@@ -150,6 +150,29 @@ def test_rows_lm_head(M_, V):
     np.testing.assert_array_equal(host(tok2, np.int32, (M_,)), t)
 
 
+# V: one group; several groups per workgroup with a shorter last one (1027 = 3 * 342 + 1)
+@pytest.mark.parametrize("V", [32, 32 * 1027])
+@pytest.mark.parametrize("M_", [1, 16, 17, 32])
+def test_rows_lm_head_ties_and_negative_rows(M_, V):
+    """Row m of x selects column m of w, so every logit is exact: the maximum of a row sits
+    at three columns (any lane, group and workgroup) and is negative in the odd rows, where
+    a padded column's zero would win."""
+    say(f"rows lm_head ties M={M_} V={V}")
+    K = 64
+    rng = np.random.default_rng(350 + M_)
+    x = np.eye(M_, K).astype(np.float16)
+    w = np.zeros((V, K), np.float16)
+    w[:, 1::2] = -2
+    want = np.zeros(M_, np.int32)
+    for m in range(M_):
+        at = rng.integers(0, V, 3)
+        w[at, m] = -1 if m % 2 else 1
+        want[m] = at.min()
+    tok = DeviceBuffer(M_ * 4)
+    ops.rows_lm_head(None, tok, dev(x), dev(w), M_, V, K, workspace=workspace(V, K))
+    np.testing.assert_array_equal(host(tok, np.int32, (M_,)), want)
+
+
 def test_rows_rejects_bad_shapes():
     say("rows: argument errors")
     from kvcache_amd import KvcError
