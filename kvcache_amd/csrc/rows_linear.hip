@@ -937,7 +937,7 @@ __global__ __launch_bounds__(kChainWaves * 64) void chain_kernel(ChainParams cp)
 }
 
 // tokens[m] = the column of the largest candidate over the workgroups (first index on
-// ties): 475 per row at 151936 outputs (one per column group, 4748, took 12 to 16 us).
+// ties): 250 per row at 151936 outputs (one per column group, 4748, took 12 to 16 us).
 constexpr int kArgThreads = 256;
 __global__ __launch_bounds__(kArgThreads) void group_argmax_kernel(const float* best_v, const int* best_i, int groups,
                                                                    int* tokens, const int* dev_rows) {
@@ -964,9 +964,9 @@ __global__ __launch_bounds__(kArgThreads) void group_argmax_kernel(const float* 
 }
 
 // ---- host side ------------------------------------------------------------------
-// Kernel shapes: (waves, k steps per wave) = (4, 7) for K <= 896 with many groups,
-// (8, 4) for K <= 1024 with few groups, (8, 4) or (4, 4) with the K range split
-// across workgroups for larger K (no prologue norm then).
+// Kernel shapes: (waves, k steps per wave) = (8, 4) for K <= 1024, (8, 4) or (4, 4)
+// with the K range split across workgroups for larger K (no prologue norm then); (4, 7)
+// for K <= 896 by tuning only.
 struct Shape {
     int groups, splits, waves, steps, gpw;
 };
@@ -977,10 +977,11 @@ Shape plan_shape(int groups, int K, bool norm) {
     const int ks = K / 32;
     Shape s{groups, 1, 4, 7, 1};
     int shape = g_tune_shape;
-    // automatic: 4x7 for very many groups (lm_head, 4748 groups: 49 us vs 51 us at
-    // 8x4), 8x4 otherwise (gate|up at I 4864, 304 groups: 7.1 us vs 7.8 us at 4x7),
-    // 8x4 with K split past 32 steps (down_proj K 4864 at 32 rows: 5 splits)
-    if (shape < 0) shape = ks <= 28 && groups >= 1024 ? 0 : ks <= 32 ? 1 : 3;
+    // automatic: 8x4 while one workgroup covers K (gate|up at I 4864, 304 groups: 7.1 us
+    // vs 7.8 us at 4x7; lm_head at 32 rows, 1536 / 3136 / 4748 / 8192 groups: 21.3 / 45.2
+    // / 64.2 / 110.2 us vs 22.3 / 47.5 / 66.8 / 114.4 us), 8x4 with K split past 32 steps
+    // (down_proj K 4864 at 32 rows: 5 splits)
+    if (shape < 0) shape = ks <= 32 ? 1 : 3;
     if (shape == 0 && ks > 28) shape = 1;
     if (shape == 1 && ks > 32) shape = 2;
     if (norm && shape >= 2) shape = 1;  // callers reject normalised K above 1024
@@ -994,12 +995,12 @@ Shape plan_shape(int groups, int K, bool norm) {
         s.splits = std::max(min_splits, g_tune_splits > 0 ? std::min(g_tune_splits, std::max(1, ks / s.waves)) : 0);
     }
     if (s.splits == 1) {
-        // groups per workgroup (measured at 32 rows): up to ~1024 groups, one workgroup
-        // per CU (256) running its groups back to back with the next one's loads in
-        // flight beats two co-resident single-group workgroups (gate/up, 304 groups:
-        // 8.7 vs 12.5 us); for many groups, about two workgroups per CU (lm_head, 4748
-        // groups: 10 per workgroup, 67-69 us, vs 78-88 us at 5-8 or 12-16)
-        const int per = groups <= 1024 ? 256 : 512;
+        // groups per workgroup (measured at 32 rows): one workgroup per CU (256) running
+        // its groups back to back with the next one's loads in flight beats two
+        // co-resident ones (gate/up, 304 groups: 8.7 vs 12.5 us; lm_head, 1536 / 3136 /
+        // 4748 groups: 21.3 / 45.2 / 64.2 us vs 26.5 / 48.9 / 66.6 us; level at 4008 and
+        // 8192, 57.2 vs 57.0 and 110.2 vs 109.9 us)
+        const int per = 256;
         s.gpw = g_tune_gpw > 0 ? g_tune_gpw : std::max(1, (groups + per - 1) / per);
     }
     return s;
