@@ -568,8 +568,11 @@ __global__ __launch_bounds__(WPB * kWave) void split_kernel(const int* __restric
         // (a short sequence of a self-planned launch: its own entries)
         constexpr bool WHOLE_TABLE = PLANNED && !LEAD;
         const int first = tab_start + (PLANNED ? 0 : b0);
+        // (a first entry outside the table must not turn the bound negative: a negative size
+        // is a descriptor over all of memory)
+        const int from = min(max(first, 0), p.table_len);
         const __amdgpu_buffer_rsrc_t trs =
-            WHOLE_TABLE ? tile_rsrc(p.table_all, min(p.table_len, first + nblk) * 4)
+            WHOLE_TABLE ? tile_rsrc(p.table_all, (from + min(nblk, p.table_len - from)) * 4)
                         : tile_rsrc(p.table_all + first, nblk * 4);
         const int tb = WHOLE_TABLE ? first * 4 : 0;  // byte offset of the chunk's first entry
         if constexpr (UNIFORM) {

@@ -325,6 +325,27 @@ def test_planned_grouped_scale_sign(orc, D, scale):
     assert np.abs(got - ref).max() <= 2e-3
 
 
+@pytest.mark.parametrize("start", [-3, -(1 << 31), 10_000, (1 << 31) - 1])
+def test_planned_table_start_outside_the_table(orc, start):
+    # a stale plan whose first table entry lies outside the table: entries past it read as 0
+    # through the table's descriptor, and the other sequences are not touched
+    say(f"planned table start={start}")
+    H, D, B = 8, 64, 16
+    lens = np.array([700, 90, 300], np.int32)
+    q, K, V = normal((3, H, D), 60, np.float32), normal((3, H, 704, D), 61, np.float32), normal((3, H, 704, D), 62, np.float32)
+    kp, vp, table, off = paged_layout(K, V, lens, B, perm=np.random.default_rng(8).permutation(80))
+    ref = orc.batched_paged(q, kp, vp, table, off, lens, H, B, 1.0 / np.sqrt(D))
+    work, nu, nr = ops.decode_plan(lens, H, H, D, B, tab_off=off, dtype=KVC_F32)
+    units = work.reshape(nu, -1)
+    units[units[:, 0] == 0, 7] = start
+    out = DeviceBuffer(q.nbytes)
+    ops.launch_batched_paged_planned(dev(q), dev(kp), dev(vp), dev(table), len(table), out, 3, H, H, D, B,
+                                     1.0 / np.sqrt(D), DeviceBuffer.from_numpy(work), nu, nr, dtype=KVC_F32)
+    got = host(out, np.float32, q.shape)
+    assert np.isfinite(got).all()
+    np.testing.assert_allclose(got[1:], ref[1:], rtol=0, atol=tol(KVC_F32))
+
+
 @pytest.mark.parametrize("lengths", ["reference", "loguniform"])
 def test_planned_c2_ragged(orc, lengths):
     lens = W.ref_lengths() if lengths == "reference" else W.loguniform_lengths(128, 16, 2048, 7)
