@@ -418,7 +418,9 @@ PlanShape plan_shape(int Hq, int Hkv, int D, int BLOCK, int dtype, int N = 0) {
         // a split costs the chunk tail a store, an arrival and a merge: sequences stay whole
         // up to 1.5 chunks of at least min_chunk_long tokens, an eighth of the longest
         // sequence between 512 (64 sequences of 128..4096 tokens 14.8 -> 13.6 us) and 1024
-        // (4 of 8192..32768: 15.3 us, 17.8 in chunks of 704), or min_chunk_long once whole
+        // (4 of 8192..32768: 15.3 us, 17.8 in chunks of 704), or min_chunk_long where that
+        // splits nothing (12 layers, 7 sequences x 4 KV heads of at most 1000 tokens: 83 us
+        // whole, 120 in chunks of at least 512: a merge for no chunk after it) and once whole
         // sequences fill the CUs (60 sequences x 8 KV heads, D 128: 23.8 us, 27.0 in chunks
         // of at least 512; 128 x 4, D 64: 15.1 and 16.1)
         auto blocks_up = [&](int x) { return (x + BLOCK - 1) / BLOCK * BLOCK; };
@@ -475,7 +477,8 @@ inline int plan_key(bool split, long long len, int T, bool split_first) {
 // tokens (the kernel's own planner applies the same rule).
 int plan_min_chunk(const PlanShape& ps, int N, int lmax, int BLOCK) {
     if (!ps.mfma) return ps.min_chunk;
-    if ((long long)N * ps.hks >= kPlanFullUnits) return std::max(ps.min_chunk, ps.min_chunk_long);
+    if ((long long)N * ps.hks >= kPlanFullUnits || lmax <= plan_whole_max(ps.min_chunk_long))
+        return std::max(ps.min_chunk, ps.min_chunk_long);
     const int eighth = (int)std::min<long long>(((long long)lmax / 8 + BLOCK - 1) / BLOCK * BLOCK, ps.min_chunk_long);
     return std::max(ps.min_chunk, eighth);
 }

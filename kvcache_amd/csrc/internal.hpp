@@ -113,6 +113,9 @@ int device_error_status(int code);
 // Grouped-query decode: with this many (sequence, KV head) pairs, one per CU, sequences are
 // only split into long chunks (plan_min_chunk).
 constexpr int kPlanFullUnits = 256;
+// ... and a batch with no longer sequence than this stays whole in chunks of at least
+// `chunk` (split_seq's rule: up to 1.5 chunks).
+constexpr long long plan_whole_max(int chunk) { return (long long)chunk * 3 / 2; }
 
 // Prompt attention with fewer keys than this is never split over workgroups: up to here
 // one workgroup's key streams take about as long as a split's partials and merge (14

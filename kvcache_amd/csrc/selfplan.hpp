@@ -224,8 +224,8 @@ __device__ SelfPlan self_plan_setup(const int* lens, int n_seq, const DecodePara
         long long T = min(c, (long long)p.sp_target_cap);
         long long least = p.sp_min_chunk;
         if constexpr (!Lds::kLead) {  // matrix cores: plan_min_chunk's rule
-            const long long eighth = (long long)N * hks >= kPlanFullUnits ? (long long)p.sp_min_long
-                                                                        : (((long long)lall >> 3) + B - 1) >> bsh << bsh;
+            const bool whole = (long long)N * hks >= kPlanFullUnits || lall <= plan_whole_max(p.sp_min_long);
+            const long long eighth = whole ? (long long)p.sp_min_long : (((long long)lall >> 3) + B - 1) >> bsh << bsh;
             least = max(least, min(eighth, (long long)p.sp_min_long));
         }
         T = max(T, least);

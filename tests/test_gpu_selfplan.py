@@ -420,3 +420,29 @@ def test_grouped_units_host_and_device_plans(orc, D, Hq, Hkv, n):
     np.testing.assert_array_equal(got, host(out, np.float16, q.shape))
     ref = orc.batched_paged(q, kp, vp, table, off, lens, Hkv, B, scale, nthreads=8)
     assert np.abs(got.astype(np.float64) - ref).max() <= tol(KVC_F16)
+
+
+@pytest.mark.parametrize("D,Hq,Hkv", [(64, 28, 4), (128, 8, 2)])
+@pytest.mark.parametrize("longest", [1000, 1536, 1537])
+def test_short_grouped_batches_stay_whole(orc, D, Hq, Hkv, longest):
+    # up to one and a half of the long chunks nothing is split (a split's merge costs more
+    # than it saves); both planners draw the line at the same length
+    say(f"short grouped batch D={D} longest={longest}")
+    lens = np.array([longest, 800, 33, 1, 700], np.int32)
+    n, B = len(lens), 16
+    nb = int(sum((int(x) + B - 1) // B for x in lens))
+    alloc = BlockAllocator(nb)
+    alloc.shuffle(longest)
+    table, off = build_tables(lens, B, alloc)
+    work, nu, nr = ops.decode_plan(lens, Hq, Hkv, D, B, tab_off=off, table=table)
+    assert (nr == 0) == (longest <= 1536)
+    kp, vp = (normal((nb, Hkv, B, D), 70 + i, np.float16) for i in range(2))
+    q = normal((n, Hq, D), 72, np.float16)
+    scale = float(1.0 / np.sqrt(D))
+    got = self_planned(q, kp, vp, table, off, lens, Hkv, B, KVC_F16)
+    out = DeviceBuffer(q.nbytes)
+    ops.launch_batched_paged_planned(dev(q), dev(kp), dev(vp), dev(table), len(table), out, n, Hq, Hkv, D, B, scale,
+                                     dev(work), nu, nr)
+    np.testing.assert_array_equal(got, host(out, np.float16, q.shape))
+    ref = orc.batched_paged(q, kp, vp, table, off, lens, Hkv, B, scale)
+    assert np.abs(got.astype(np.float64) - ref).max() <= tol(KVC_F16)
