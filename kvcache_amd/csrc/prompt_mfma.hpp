@@ -38,7 +38,45 @@
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
 
+// Inf and NaN in V behind the causal edge.  A key that a query does not see has probability
+// 0, and 0 x Inf is NaN, so in the tiles of the edge the elements of V that are not finite
+// are staged as 0 (clear_nonfinite) and a workgroup that met one adds them, in its epilogue,
+// to the queries that see their key (add_nonfinite).
+__device__ __forceinline__ bool nonfinite(unsigned half_bits) { return (half_bits & 0x7C00u) == 0x7C00u; }
+
+// Clears the halves of v that are Inf or NaN; true if there were any in the wave.
+template <int NV>
+__device__ __forceinline__ bool clear_nonfinite(u32x4 (&v)[NV]) {
+    unsigned c = 0;  // an exponent of all ones carries into its half's top bit
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c |= (v[i][e] & 0x7C007C00u) + 0x04000400u;
+    if (!__any((c & 0x80008000u) != 0)) return false;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            v[i][e] &= (nonfinite(v[i][e]) ? 0u : 0xFFFFu) | (nonfinite(v[i][e] >> 16) ? 0u : 0xFFFF0000u);
+    return true;
+}
+
+// acc += the elements d0 .. d0 + 3 of V that are Inf or NaN, of keys [first, last].
+template <int D>
+__device__ __forceinline__ f32x4 add_nonfinite(f32x4 acc, const char* vb, const int* table, int bsh, int Hkv, int hk,
+                                            int first, int last, int d0) {
+    for (int j = first; j <= last; ++j) {
+        const size_t row = ((size_t)(unsigned)(table[j >> bsh] * Hkv + hk) << bsh) + (j & ((1 << bsh) - 1));
+        const f16x4 v = *reinterpret_cast<const f16x4*>(vb + (row * D + d0) * 2);
+        const u16x4 bits = __builtin_bit_cast(u16x4, v);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (nonfinite(bits[r])) acc[r] += (float)v[r];
+    }
+    return acc;
+}
 
 template <int D, int QG, int W>
 __global__ __launch_bounds__(W * kWave) void prompt_kernel(DecodeParams p) {
@@ -53,6 +91,7 @@ __global__ __launch_bounds__(W * kWave) void prompt_kernel(DecodeParams p) {
     constexpr int kSetBytes = kPromptSet * ROW;
     __shared__ __attribute__((aligned(16))) char s_kv[2][2][kSetBytes];  // [half][K / V]
     __shared__ float s_ml[KS][QG][32][2];
+    __shared__ int s_bad[W];
     static_assert(KS * QG * 32 * D * 4 <= 2 * 2 * kSetBytes, "partials fit the tile buffers");
 
     const int lane = threadIdx.x & (kWave - 1);
@@ -70,6 +109,8 @@ __global__ __launch_bounds__(W * kWave) void prompt_kernel(DecodeParams p) {
     const int base = p.fixed_len;
     const int lmax = base + min(q0 + 32 * QG, p.N);  // keys of the tile's last query
     const int nsets = (lmax + kPromptSet - 1) / kPromptSet;
+    const int nfull = min(nsets, (base + q0 + 1) / kPromptSet);  // sets that every query of the tile sees whole
+    bool bad = false;  // this wave cleared elements of V in the sets after those
     const int qw = q0 + 32 * qg;                     // the wave's first query
     const int qlast = base + qw + l32;               // last key this column sees
 
@@ -103,7 +144,8 @@ __global__ __launch_bounds__(W * kWave) void prompt_kernel(DecodeParams p) {
     };
     auto kchunk = [](int r, int ch) { return ch ^ (r & 7); };
     auto vseg = [](int r, int seg) { return seg ^ (D == 64 ? (r >> 1) & 3 : r & 7); };
-    auto store = [&](int half) {
+    auto store = [&](int half, bool edge) {
+        if (edge) bad |= clear_nonfinite(rv);
 #pragma unroll
         for (int i = 0; i < VL; ++i) {
             const int off = i * 1024 + lane * 16;
@@ -210,23 +252,21 @@ __global__ __launch_bounds__(W * kWave) void prompt_kernel(DecodeParams p) {
     };
 
     const int wlast = base + min(qw + 31, p.N - 1);  // last key any query of the wave sees
-    store(0);
+    store(0, nfull == 0);
     issue_k(1);
     issue_v();
     // one set: the next one from its registers into the other half of the buffer, the
     // one after that into flight, then this one's arithmetic
     auto set = [&](int s, auto masked_tag) {
         __syncthreads();
-        store((s + 1) & 1);
+        store((s + 1) & 1, decltype(masked_tag)::value || s + 1 >= nfull);
         if (((s + 2) & (kWave - 1)) == 0) load_ids(s + 2);
         issue_k(s + 2);  // (sets past the end read nothing: zero-size descriptors)
         issue_v();
         const int t0 = s * kPromptSet + ks * KT;
         if (!decltype(masked_tag)::value || (qw < p.N && t0 <= wlast)) compute(s & 1, t0, masked_tag);
     };
-    // sets that every query of the tile sees whole, then those with the causal edge (in
-    // loops of their own: one loop with both forms copied O between them in every set)
-    const int nfull = min(nsets, (base + q0 + 1) / kPromptSet);
+    // (loops of their own: one loop with both forms copied O between them in every set)
     int s = 0;
     for (; s < nfull; ++s) set(s, std::false_type{});
     for (; s < nsets; ++s) set(s, std::true_type{});
@@ -248,6 +288,7 @@ __global__ __launch_bounds__(W * kWave) void prompt_kernel(DecodeParams p) {
         s_ml[ks][qg][l32][0] = m;
         s_ml[ks][qg][l32][1] = l;
     }
+    if (lane == 0) s_bad[wave] = bad;
     __syncthreads();
     float M = -FLT_MAX;
 #pragma unroll
@@ -269,6 +310,14 @@ __global__ __launch_bounds__(W * kWave) void prompt_kernel(DecodeParams p) {
     }
     const int q = qw + l32;
     if (q >= p.N) return;
+    int any_bad = 0;
+#pragma unroll
+    for (int w = 0; w < W; ++w) any_bad |= s_bad[w];
+    if (any_bad)
+#pragma unroll
+        for (int i = 0; i < SL; ++i)
+            acc[i] = add_nonfinite<D>(acc[i], vb, p.table_all, bsh, p.Hkv, hk, nfull * kPromptSet, qlast,
+                                      8 * (ks * SL + i) + 4 * h);
     const float inv = lt > 0.f ? 1.0f / lt : 0.f;
     _Float16* ob = static_cast<_Float16*>(p.out) + ((size_t)q * p.Hq + qh) * D + 4 * h;
 #pragma unroll
@@ -293,6 +342,7 @@ __global__ __launch_bounds__(8 * kWave) void prompt_stream_kernel(DecodeParams p
     constexpr int kTile = 32 * ROW;          // bytes of one K (or V) tile
     __shared__ __attribute__((aligned(16))) char s_kv[W][2][kTile];
     __shared__ float s_ml[W][32 * NC][2];
+    __shared__ int s_bad[W];
 
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = uniform(threadIdx.x >> 6);
@@ -461,7 +511,9 @@ __global__ __launch_bounds__(8 * kWave) void prompt_stream_kernel(DecodeParams p
                 for (int n = 0; n < NC; ++n) O[n][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb[n][t], O[n][dt], 0, 0, 0);
             }
     };
+    bool bad = false;  // this wave cleared elements of V in its tiles of the causal edge
     auto step = [&](int k, auto masked_tag) {
+        if constexpr (decltype(masked_tag)::value) bad |= clear_nonfinite(rv[0]) | clear_nonfinite(rv[1]);
         __builtin_amdgcn_wave_barrier();
         stage();
         __builtin_amdgcn_wave_barrier();
@@ -485,6 +537,7 @@ __global__ __launch_bounds__(8 * kWave) void prompt_stream_kernel(DecodeParams p
     static_assert(kSlots % W == 0 && W * kSlots * kWave * 16 <= (int)sizeof(s_kv), "the partials fit the tiles");
     f32x4* part = reinterpret_cast<f32x4*>(&s_kv[0][0][0]);
     __syncthreads();
+    if (lane == 0) s_bad[wave] = bad;
 #pragma unroll
     for (int n = 0; n < NC; ++n) {
         const float lt = sum_xor32(l[n]);
@@ -523,6 +576,14 @@ __global__ __launch_bounds__(8 * kWave) void prompt_stream_kernel(DecodeParams p
     }
     const int q = q0 + col;
     const int ncq = max(base + q, 0) / chunk + 1;  // chunks of the query
+    int any_bad = 0;
+#pragma unroll
+    for (int w = 0; w < W; ++w) any_bad |= s_bad[w];
+    if (any_bad)
+#pragma unroll
+        for (int i = 0; i < kPer; ++i)
+            acc[i] = add_nonfinite<D>(acc[i], vb, p.table_all, bsh, p.Hkv, hk, j0 + 32 * full, min(base + q, j1 - 1),
+                                      8 * ((wave * kPer + i) % (DT * 4)) + 4 * h);
     // host positions: merge_kernel follows (20 queries, 14 heads, behind 5900 keys: 10.5 us,
     // 13.9 merged in here); a device position does not know on the host whether one is needed
     const bool fused = p.merge_mode == kMergeAtomic;

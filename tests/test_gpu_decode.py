@@ -511,6 +511,44 @@ def test_prompt_tiles(orc, D, Hq, Hkv, B, base, n, device_pos):
     assert np.abs(got - want).max() <= tol(KVC_F16)
 
 
+# the edge tiles of every prompt kernel: 32, 64 and 128 queries, split and not, the position on
+# the host and on the device (from 8 grouped queries on)
+@pytest.mark.parametrize("D,Hq,Hkv,base,n,device_pos", [
+    (64, 14, 2, 5, 40, False), (64, 14, 2, 5, 40, True), (64, 14, 2, 3500, 33, False), (64, 14, 2, 3500, 33, True),
+    (64, 14, 2, 40, 9, False), (64, 128, 4, 0, 255, False), (128, 8, 2, 127, 32, False), (128, 8, 2, 4100, 40, True),
+    (128, 64, 2, 16, 150, False), (128, 64, 2, 0, 257, False)])
+def test_prompt_nonfinite_values_reach_only_later_queries(orc, D, Hq, Hkv, base, n, device_pos):
+    """Inf and NaN in V at a key: queries before it are those of a finite V, later ones are not
+    finite in just the dims it touches."""
+    say(f"prompt non-finite V D={D} Hq={Hq} Hkv={Hkv} base={base} n={n} device_pos={device_pos}")
+    B = 16
+    nb = (base + n + B - 1) // B
+    table = np.random.default_rng(base + n).permutation(nb + 3)[:nb].astype(np.int32)
+    kp, vp = normal((nb + 3, Hkv, B, D), 220, np.float16), normal((nb + 3, Hkv, B, D), 221, np.float16)
+    q = normal((n, Hq, D), 222, np.float16)
+    bad = np.zeros((n, Hkv, D), bool)  # [query]: dims that a key it sees has made non-finite
+    finite = vp.copy()
+    for at, hk, dims, x in ((n // 3, 0, slice(None), np.inf), (2 * n // 3, Hkv - 1, slice(3, 4), np.nan),
+                            (n - 2, Hkv - 1, slice(D - 1, D), -np.inf)):
+        j = base + at
+        vp[table[j // B], hk, j % B, dims] = x
+        finite[table[j // B], hk, j % B, dims] = 0
+        bad[at:, hk, dims] = True
+    scale = float(1.0 / np.sqrt(D))
+    out = DeviceBuffer(q.nbytes)
+    if device_pos:
+        ops.qkcuda_paged_causal_attn(dev(q), out, dev(kp), dev(vp), dev(table), dev(np.array([base], np.int32)), n, Hq,
+                                     Hkv, D, B, scale)
+    else:
+        ops.qk_paged_causal_attn(dev(q), out, dev(kp), dev(vp), dev(table), base, n, Hq, Hkv, D, B, scale)
+    got = host(out, np.float16, q.shape).astype(np.float64)
+    want = orc.paged_causal(q, kp, finite, table, base, Hkv, B, scale, nthreads=8)
+    bad = np.repeat(bad, Hq // Hkv, axis=1)
+    assert not np.isfinite(got[bad]).any()
+    assert np.isfinite(got[~bad]).all()
+    assert np.abs(got - want)[~bad].max() <= tol(KVC_F16)
+
+
 def test_prefill_flow_write_then_causal_attn(orc):
     """The model path's prefill (qwen_serve.cu:106-108): write the P prompt rows of
     K/V through the sequence's table, then causal attention over them."""
