@@ -881,12 +881,13 @@ int run_self_planned(const void* q, const void* k, const void* v, const int* tab
     if (cap > 0) upper = std::min(upper, (long long)ps.hks * N * ((long long)cap / std::max(ps.min_chunk, 1) + 2));
     if (tuning().self_grid > 0) upper = std::min(upper, (long long)tuning().self_grid);
     L.units = (int)std::min<long long>(std::max(upper, 1LL), INT_MAX);
-    // prompt queries at a device position: prompt_stream_kernel, whose tiles share their
-    // keys' loads (14q/2kv, 96 queries behind 1500 keys 14.2 -> 10.9 us, 400 behind 4000
-    // 87 -> 21 us; 8 heads, one query behind 1500 10.9 -> 9.9 us).  Up to 7 queries of
-    // grouped heads stay with the decode units, which read each key once for the group: at
-    // 60000 keys and one query 18 us against 25 (at 4000, 15.4 against 9.5)
-    if (!contig && !cur_len && (N >= 8 || !ps.mfma) && causal_tile_path(N, Hq, Hkv, D, BLOCK, dtype) &&
+    // prompt queries of grouped heads at a device position: prompt_stream_kernel, whose tiles
+    // share their keys' loads (14q/2kv, 96 queries behind 1500 keys 14.2 -> 10.9 us, 400
+    // behind 4000 87 -> 21 us).  Up to 7 queries stay with the decode units, which read each
+    // key once for the group: at 60000 keys and one query 18 us against 25 (at 4000, 15.4
+    // against 9.5).  Heads that are not grouped stay as well: their units (split_kernel) keep
+    // the probabilities in 32 bits, prompt_stream_kernel rounds them to 16 for the matrix cores
+    if (!contig && !cur_len && N >= 8 && ps.mfma && causal_tile_path(N, Hq, Hkv, D, BLOCK, dtype) &&
         (long long)((N + 31) / 32) * Hq <= recs) {
         L.mode = kCausalTile;
         L.mfma = true;

@@ -549,6 +549,28 @@ def test_prompt_nonfinite_values_reach_only_later_queries(orc, D, Hq, Hkv, base,
     assert np.abs(got - want)[~bad].max() <= tol(KVC_F16)
 
 
+@pytest.mark.parametrize("D,Hq,Hkv", [(64, 8, 8), (64, 12, 4), (128, 8, 4), (64, 17, 1)])
+@pytest.mark.parametrize("n", [1, 9])
+def test_device_position_keeps_probabilities_in_32_bits(orc, D, Hq, Hkv, n):
+    """Heads in groups the matrix-core units do not take (1 to 3 and above 16 per KV head): the
+    arithmetic is fp32 throughout, so the only 16-bit rounding is the output's.  An error of
+    1e-6 moves a rounding in about 1e-6 / 2^-11 = 0.2% of the values, probabilities of 16 bits
+    (2e-4) in a third of them."""
+    say(f"device position, 32-bit probabilities D={D} Hq={Hq} Hkv={Hkv} n={n}")
+    B, base = 16, 700
+    nb = (base + n + B - 1) // B
+    table = np.random.default_rng(n).permutation(nb).astype(np.int32)
+    kp, vp = normal((nb, Hkv, B, D), 230, np.float16), normal((nb, Hkv, B, D), 231, np.float16)
+    q = normal((n, Hq, D), 232, np.float16)
+    scale = float(1.0 / np.sqrt(D))
+    out = DeviceBuffer(q.nbytes)
+    ops.qkcuda_paged_causal_attn(dev(q), out, dev(kp), dev(vp), dev(table), dev(np.array([base], np.int32)), n, Hq, Hkv,
+                                 D, B, scale)
+    got = host(out, np.float16, q.shape)
+    want = orc.paged_causal(q, kp, vp, table, base, Hkv, B, scale)
+    assert np.mean(got != want.astype(np.float16)) <= 0.02
+
+
 def test_prefill_flow_write_then_causal_attn(orc):
     """The model path's prefill (qwen_serve.cu:106-108): write the P prompt rows of
     K/V through the sequence's table, then causal attention over them."""
