@@ -642,7 +642,7 @@ int prompt_qtile(int Nq, int Hq, int D) {
 // 14 heads behind 20000 keys: 13.6 us with up to 256 workgroups, 15.5 with 128, 16.9 with
 // 512; 20 queries of 32 heads, D 128, behind 5900: 22.2 us in chunks of 1024, 26 of 1536).
 int prompt_max_chunks(int Nq, int Hq) {
-    const long long wgs = (long long)((Nq + 31) / 32) * Hq;
+    const long long wgs = std::max(1LL, (long long)((Nq + 31) / 32) * Hq);
     return (int)std::min(64LL, std::max(1LL, 256 / wgs));
 }
 int prompt_min_chunk(int D) { return D == 64 ? 512 : 1024; }

@@ -321,3 +321,11 @@ def test_decode_plan_chunk_sizing():
         work, nu, nr = ops.decode_plan(lens, Hq, Hkv, 64, 16, dtype=KVC_F16)
         sizes = work[:, 3] - work[:, 2]
         assert nu == units and sizes.max() <= biggest, (nu, int(sizes.max()))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_prompt_workspace_of_no_queries(D):
+    # no queries behind a long prefix: a size, not a division by the zero tiles
+    from kvcache_amd._native import lib
+    for base in (0, 4000, 2**31 - 1):
+        assert lib().kvc_paged_causal_attn_workspace_size(base, 0, 14, 2, D, 16, KVC_F16) == 0
