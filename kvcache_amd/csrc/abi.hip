@@ -638,14 +638,29 @@ int prompt_qtile(int Nq, int Hq, int D) {
 }
 
 // Chunks a tile's keys may be split into (32-query tiles only: few workgroups, long
-// prefixes): up to one workgroup per CU, of at least prompt_min_chunk keys (one query of
-// 14 heads behind 20000 keys: 13.6 us with up to 256 workgroups, 15.5 with 128, 16.9 with
-// 512; 20 queries of 32 heads, D 128, behind 5900: 22.2 us in chunks of 1024, 26 of 1536).
+// prefixes): up to one workgroup per CU (one query of 14 heads behind 20000 keys: 13.6 us
+// with up to 256 workgroups, 15.5 with 128, 16.9 with 512).
 int prompt_max_chunks(int Nq, int Hq) {
     const long long wgs = std::max(1LL, (long long)((Nq + 31) / 32) * Hq);
     return (int)std::min(64LL, std::max(1LL, 256 / wgs));
 }
+// Position in device memory: least keys per chunk (the kernel splits, prompt_mfma.hpp).
 int prompt_min_chunk(int D) { return D == 64 ? 512 : 1024; }
+
+// Position on the host: rounds of 256 keys (a 32-key tile per wave) in a chunk, of the
+// `rounds` that the longest tile has.  Rounds cost 0.83 us each (head_dim 128: 1.33), the
+// partials and the merge kernel 2.5 us and another 1 per 400 (query, head) rows (14 rows 2.5
+// us, 462 4.1, 1024 5.2, 2048 7.8, 4096 13), so a split has to save more rounds than that.
+// Behind 2900 keys, whole -> split: one query of 14 heads 14.8 -> 8.5 us, of 32 heads, D 128,
+// 21.8 -> 11.7, 33 queries of 14 heads 15.6 -> 11.1; 128 queries of 32 heads behind 4000, D
+// 64: 20.1 whole, 27.3 in two.  One query behind 800: 7.6 whole, 8.4 split.
+int prompt_chunk_rounds(int rounds, int Nq, int Hq, int D) {
+    const int nch = prompt_max_chunks(Nq, Hq);
+    const int r = (rounds + nch - 1) / nch;
+    const long long rows = (long long)Nq * Hq;
+    const long long cost = D == 64 ? 3 + rows / 256 : 2 + rows / 448;
+    return rounds - r > cost ? r : rounds;
+}
 
 Plan plan_causal_tile(int base, int Nq, int Hq, int Hkv, int D, int BLOCK) {
     Plan pl;
@@ -656,11 +671,10 @@ Plan plan_causal_tile(int base, int Nq, int Hq, int Hkv, int D, int BLOCK) {
     pl.wpb = 8;
     pl.qtile = prompt_qtile(Nq, Hq, D);
     const long long lmax = std::max(1LL, (long long)base + Nq);
-    long long nch = 1;
-    if (pl.qtile == 32 && lmax >= kPromptSplitMin)
-        nch = std::min<long long>(prompt_max_chunks(Nq, Hq), std::max(1LL, lmax / prompt_min_chunk(D)));
+    long long rounds = (lmax + 255) / 256;
+    if (pl.qtile == 32) rounds = prompt_chunk_rounds((int)rounds, Nq, Hq, D);
     const long long al = std::max(BLOCK, 256);
-    const long long ch = std::min<long long>((lmax + nch * al - 1) / (nch * al) * al, INT_MAX);
+    const long long ch = std::min<long long>((rounds * 256 + al - 1) / al * al, INT_MAX);
     pl.chunk = (int)ch;
     pl.max_chunks = (int)((lmax + ch - 1) / ch);
     size_workspace(pl, Nq, Hq, Hkv, D);

@@ -117,9 +117,10 @@ constexpr int kPlanFullUnits = 256;
 // `chunk` (split_seq's rule: up to 1.5 chunks).
 constexpr long long plan_whole_max(int chunk) { return (long long)chunk * 3 / 2; }
 
-// Prompt attention with fewer keys than this is never split over workgroups: up to here
-// one workgroup's key streams take about as long as a split's partials and merge (14
-// heads, D 64: 100 queries behind 2000 tokens 12.2 us whole, 13.5 us in chunks of 512).
+// Prompt attention at a device position with fewer keys than this is never split over
+// workgroups: up to here one workgroup's key streams take about as long as a split's partials
+// and its merge in the launch (14 heads, D 64: 100 queries behind 2000 tokens 12.2 us whole,
+// 13.5 us in chunks of 512).
 constexpr int kPromptSplitMin = 3072;
 
 // Arrival counters.  Atomics that land on one 128-byte line serialise (about 10 ns

@@ -329,3 +329,23 @@ def test_prompt_workspace_of_no_queries(D):
     from kvcache_amd._native import lib
     for base in (0, 4000, 2**31 - 1):
         assert lib().kvc_paged_causal_attn_workspace_size(base, 0, 14, 2, D, 16, KVC_F16) == 0
+
+
+def test_prompt_split_follows_the_rounds_it_saves():
+    # a split is paid for with its partials and merge (2.5 us and more per (query, head) row), so
+    # few queries behind a long prefix are split and many are not; without a split no workspace
+    from kvcache_amd._native import lib
+
+    def chunks(base, nq, hq, hkv, D):
+        n = lib().kvc_paged_causal_attn_workspace_size(base, nq, hq, hkv, D, 16, KVC_F16)
+        return round(n / (nq * hq * (D + 2) * 4)) if n else 1
+
+    assert chunks(800, 1, 14, 2, 64) == 1
+    for base in (1500, 2900, 4000):  # one tile per wave
+        assert chunks(base, 1, 14, 2, 64) == (base + 256) // 256
+        assert chunks(base, 16, 8, 8, 64) >= (base + 256) // 256
+    assert chunks(800, 1, 32, 8, 128) == 4
+    assert chunks(2900, 33, 14, 2, 64) == 6
+    assert chunks(2900, 33, 32, 8, 128) == 4
+    assert chunks(4000, 128, 32, 8, 64) == 1  # 4096 rows to merge: 20 us whole, 27 in two
+    assert chunks(2900, 700, 14, 2, 64) == 1
