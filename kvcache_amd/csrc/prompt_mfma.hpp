@@ -46,21 +46,29 @@ typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
 // to the queries that see their key (add_nonfinite).
 __device__ __forceinline__ bool nonfinite(unsigned half_bits) { return (half_bits & 0x7C00u) == 0x7C00u; }
 
-// Clears the halves of v that are Inf or NaN; true if there were any in the wave.
+// Whether the wave's v hold Inf or NaN.
 template <int NV>
-__device__ __forceinline__ bool clear_nonfinite(u32x4 (&v)[NV]) {
-    unsigned c = 0;  // an exponent of all ones carries into its half's top bit
+__device__ __forceinline__ bool any_nonfinite(const u32x4 (&v)[NV]) {
+    const f16x2 zero = {(_Float16)0.f, (_Float16)0.f};
+    f16x2 c[4] = {zero, zero, zero, zero};  // + x * 0: stays 0 unless some x is Inf or NaN
 #pragma unroll
     for (int i = 0; i < NV; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) c |= (v[i][e] & 0x7C007C00u) + 0x04000400u;
-    if (!__any((c & 0x80008000u) != 0)) return false;
+        for (int e = 0; e < 4; ++e) {
+            const unsigned x = v[i][e];
+            c[e] = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, x), zero, c[e]);
+        }
+    const f16x2 t = (c[0] + c[1]) + (c[2] + c[3]);
+    return __any(!(t[0] == zero[0] && t[1] == zero[1]));
+}
+
+template <int NV>
+__device__ __forceinline__ void clear_nonfinite(u32x4 (&v)[NV]) {
 #pragma unroll
     for (int i = 0; i < NV; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             v[i][e] &= (nonfinite(v[i][e]) ? 0u : 0xFFFFu) | (nonfinite(v[i][e] >> 16) ? 0u : 0xFFFF0000u);
-    return true;
 }
 
 // acc += the elements d0 .. d0 + 3 of V that are Inf or NaN, of keys [first, last].
@@ -145,7 +153,10 @@ __global__ __launch_bounds__(W * kWave) void prompt_kernel(DecodeParams p) {
     auto kchunk = [](int r, int ch) { return ch ^ (r & 7); };
     auto vseg = [](int r, int seg) { return seg ^ (D == 64 ? (r >> 1) & 3 : r & 7); };
     auto store = [&](int half, bool edge) {
-        if (edge) bad |= clear_nonfinite(rv);
+        if (edge && any_nonfinite(rv)) {
+            clear_nonfinite(rv);
+            bad = true;
+        }
 #pragma unroll
         for (int i = 0; i < VL; ++i) {
             const int off = i * 1024 + lane * 16;
@@ -334,7 +345,7 @@ __global__ __launch_bounds__(W * kWave) void prompt_kernel(DecodeParams p) {
 // barrier holds the waves in step (where every wave meets the same unit at once: loads,
 // then LDS writes, then MFMAs) and a K/V fragment read from LDS serves NC column tiles.
 template <int D, int NC>
-__global__ __launch_bounds__(8 * kWave) void prompt_stream_kernel(DecodeParams p) {
+__global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kernel(DecodeParams p) {
     constexpr int ROW = D * 2;
     constexpr int KD = D / 16, DT = D / 32;
     constexpr int VL = 16 * ROW / 1024;      // wave loads per 16-row subtile
@@ -342,7 +353,6 @@ __global__ __launch_bounds__(8 * kWave) void prompt_stream_kernel(DecodeParams p
     constexpr int kTile = 32 * ROW;          // bytes of one K (or V) tile
     __shared__ __attribute__((aligned(16))) char s_kv[W][2][kTile];
     __shared__ float s_ml[W][32 * NC][2];
-    __shared__ int s_bad[W];
 
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = uniform(threadIdx.x >> 6);
@@ -513,9 +523,16 @@ __global__ __launch_bounds__(8 * kWave) void prompt_stream_kernel(DecodeParams p
     };
     bool bad = false;  // this wave cleared elements of V in its tiles of the causal edge
     auto step = [&](int k, auto masked_tag) {
-        if constexpr (decltype(masked_tag)::value) bad |= clear_nonfinite(rv[0]) | clear_nonfinite(rv[1]);
         __builtin_amdgcn_wave_barrier();
         stage();
+        if constexpr (decltype(masked_tag)::value) {  // (while the LDS writes are under way)
+            if (any_nonfinite(rv[0]) | any_nonfinite(rv[1])) {
+                clear_nonfinite(rv[0]);
+                clear_nonfinite(rv[1]);
+                bad = true;
+                stage();
+            }
+        }
         __builtin_amdgcn_wave_barrier();
         asm volatile("" ::: "memory");
         if (((2 * (k + 1)) & (kWave - 1)) == 0) load_ids(2 * (k + 1));
@@ -537,48 +554,55 @@ __global__ __launch_bounds__(8 * kWave) void prompt_stream_kernel(DecodeParams p
     static_assert(kSlots % W == 0 && W * kSlots * kWave * 16 <= (int)sizeof(s_kv), "the partials fit the tiles");
     f32x4* part = reinterpret_cast<f32x4*>(&s_kv[0][0][0]);
     __syncthreads();
-    if (lane == 0) s_bad[wave] = bad;
+    const int nw = min(W, ntiles);  // waves that had tiles
+    if (wave < max(nw, 2) || nw > 2) {
 #pragma unroll
-    for (int n = 0; n < NC; ++n) {
-        const float lt = sum_xor32(l[n]);
-        if (h == 0) {
-            s_ml[wave][32 * n + l32][0] = m[n];
-            s_ml[wave][32 * n + l32][1] = lt;
+        for (int n = 0; n < NC; ++n) {
+            const float lt = sum_xor32(l[n]);
+            if (h == 0) {
+                s_ml[wave][32 * n + l32][0] = m[n];
+                s_ml[wave][32 * n + l32][1] = bad ? -lt : lt;  // (the sign, also of 0: elements to add)
+            }
+#pragma unroll
+            for (int i = 0; i < DT * 4; ++i)
+                part[((wave * NC + n) * DT * 4 + i) * kWave + lane] =
+                    f32x4{O[n][i >> 2][4 * (i & 3)], O[n][i >> 2][4 * (i & 3) + 1], O[n][i >> 2][4 * (i & 3) + 2],
+                          O[n][i >> 2][4 * (i & 3) + 3]};
         }
-#pragma unroll
-        for (int i = 0; i < DT * 4; ++i)
-            part[((wave * NC + n) * DT * 4 + i) * kWave + lane] =
-                f32x4{O[n][i >> 2][4 * (i & 3)], O[n][i >> 2][4 * (i & 3) + 1], O[n][i >> 2][4 * (i & 3) + 2],
-                      O[n][i >> 2][4 * (i & 3) + 3]};
     }
     __syncthreads();
     const int n = NC == 1 ? 0 : wave * kPer / (DT * 4), col = 32 * n + l32;
-    float M = -FLT_MAX, mw[W];
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-        mw[w] = s_ml[w][col][0];
-        M = fmaxf(M, mw[w]);
-    }
-    float lt = 0.f;
+    float M = -FLT_MAX, lt = 0.f;
+    unsigned any_bad = 0;
     f32x4 acc[kPer];
 #pragma unroll
     for (int i = 0; i < kPer; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto combine = [&](auto n_tag) {
+        constexpr int NW = decltype(n_tag)::value;
+        float mw[NW];
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-        const float wk = fast_exp2(mw[w] - M);
-        lt = __builtin_fmaf(wk, s_ml[w][col][1], lt);
-#pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-            const f32x4 x = part[(w * kSlots + wave * kPer + i) * kWave + lane];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[i][r] = __builtin_fmaf(wk, x[r], acc[i][r]);
+        for (int w = 0; w < NW; ++w) {
+            mw[w] = s_ml[w][col][0];
+            M = fmaxf(M, mw[w]);
         }
-    }
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const float wk = fast_exp2(mw[w] - M), lw = s_ml[w][col][1];
+            any_bad |= __float_as_uint(lw) & 0x80000000u;
+            lt = __builtin_fmaf(wk, fabsf(lw), lt);
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) {
+                const f32x4 x = part[(w * kSlots + wave * kPer + i) * kWave + lane];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[i][r] = __builtin_fmaf(wk, x[r], acc[i][r]);
+            }
+        }
+    };
+    // prompts of up to 64 keys leave two waves' partials (8 queries: 5.0 us with all eight, 4.5)
+    if (nw > 2) combine(std::integral_constant<int, W>{});
+    else combine(std::integral_constant<int, 2>{});
     const int q = q0 + col;
     const int ncq = max(base + q, 0) / chunk + 1;  // chunks of the query
-    int any_bad = 0;
-#pragma unroll
-    for (int w = 0; w < W; ++w) any_bad |= s_bad[w];
     if (any_bad)
 #pragma unroll
         for (int i = 0; i < kPer; ++i)
