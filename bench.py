@@ -584,7 +584,7 @@ def bench_c3(steps, warmup, plan_sweep=()):
     try:
         t_probe, nu_probe = practical_ceiling(W, lens, Hq, Hkv, D, B, steps, warmup, target=512)
     finally:
-        set_tuning("mfma_min_chunk", 1024)
+        set_tuning("mfma_min_chunk", 0)
     res["roofline"]["practical_ceiling_us"] = round(t_probe, 3)
     res["roofline"]["practical_ceiling"] = {
         "what": "kvc_read_probe_planned over 512-token units of every (sequence, KV head): the split kernel's "

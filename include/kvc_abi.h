@@ -72,7 +72,8 @@ int         kvc_device_count(int* count);
  * "wg_per_cu" (cap on decode workgroups per CU through reserved LDS: -1
  * automatic, 0 none, n), "split_first" (planner: chunks of split sequences
  * before whole sequences), "mfma_min_chunk" (planner, grouped-query heads on the
- * matrix cores: tokens below which a sequence stays in one unit, default 1024),
+ * matrix cores: tokens below which a sequence stays in one unit; default 0: by the
+ * batch, 256 to 1024),
  * "self_plan" (device-length decode with the automatic split: 1 = the kernel
  * derives the planner's units from the device lengths, 0 = a chunk x sequence x
  * head grid sized by cap), "self_grid" (self-planned launches: 0 = one workgroup

@@ -424,8 +424,10 @@ PlanShape plan_shape(int Hq, int Hkv, int D, int BLOCK, int dtype, int N = 0) {
         // sequences fill the CUs (60 sequences x 8 KV heads, D 128: 23.8 us, 27.0 in chunks
         // of at least 512; 128 x 4, D 64: 15.1 and 16.1)
         auto blocks_up = [&](int x) { return (x + BLOCK - 1) / BLOCK * BLOCK; };
-        ps.min_chunk = blocks_up(std::min(tuning().mfma_min_chunk, 512));
-        ps.min_chunk_long = blocks_up(tuning().mfma_min_chunk);
+        // a stated mfma_min_chunk is the least chunk of every batch
+        const int stated = tuning().mfma_min_chunk;
+        ps.min_chunk = blocks_up(stated > 0 ? stated : 512);
+        ps.min_chunk_long = blocks_up(stated > 0 ? stated : 1024);
         ps.max_chunk = kMfmaMaxChunkBlocksHost * BLOCK;
         // units to aim for: one per CU for head_dim 64; for 128 about two, whose shorter
         // chunks balance the rounds of a large batch (200 sequences, device lengths: 172
@@ -1499,7 +1501,7 @@ int kvc_set_tuning(const char* key, int value) {
     else if (k == "mfma" && value >= -1 && value <= 1) tuning().mfma = value;
     else if (k == "wg_per_cu" && value >= -1 && value <= 32) tuning().wg_per_cu = value;
     else if (k == "split_first" && (value == 0 || value == 1)) tuning().split_first = value;
-    else if (k == "mfma_min_chunk" && value >= 16 && value <= 1 << 20) tuning().mfma_min_chunk = value;
+    else if (k == "mfma_min_chunk" && (value == 0 || (value >= 16 && value <= 1 << 20))) tuning().mfma_min_chunk = value;
     else if (k == "self_plan" && (value == 0 || value == 1)) tuning().self_plan = value;
     else if (k == "self_grid" && value >= 0) tuning().self_grid = value;
     else if (k == "self_prefetch_kib" && value >= 0) tuning().self_prefetch_kib = value;

@@ -190,7 +190,8 @@ struct Tuning {
     int wg_per_cu = -1;         // >0: reserve LDS so at most this many decode workgroups share a CU;
                                 // 0: no cap; -1: automatic (4 on the planned one/two-head path)
     int split_first = 1;        // planner: chunks of split sequences before whole sequences
-    int mfma_min_chunk = 1024;  // planner, grouped-query path: tokens below which a sequence stays in one unit
+    int mfma_min_chunk = 0;     // planner, grouped-query path: tokens below which a sequence stays in one unit
+                                // (0: by the batch, plan_shape)
     int self_plan = 1;          // device-length decode with an automatic split: 1 the kernel plans its own
                                 // units (selfplan.hpp), 0 the chunk x sequence x head grid
     int self_grid = 0;          // self-planned launches: 0 automatic (resident workgroups), n: at most n

@@ -349,3 +349,26 @@ def test_prompt_split_follows_the_rounds_it_saves():
     assert chunks(2900, 33, 32, 8, 128) == 4
     assert chunks(4000, 128, 32, 8, 64) == 1  # 4096 rows to merge: 20 us whole, 27 in two
     assert chunks(2900, 700, 14, 2, 64) == 1
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_stated_min_chunk_keeps_shorter_sequences_whole(D):
+    # the tuning key "mfma_min_chunk": no sequence of at most that many tokens is split, whatever
+    # else is in the batch; 0 (the default) chooses by the batch
+    import ctypes as C
+
+    from _helpers import tuning
+    from kvcache_amd import ops
+    from kvcache_amd._native import lib
+    lens = np.array([15000, 5000, 1600, 900, 700, 30], np.int32)
+    v = C.c_int(-1)
+    assert lib().kvc_get_tuning(b"mfma_min_chunk", C.byref(v)) == 0 and v.value == 0
+    for stated in (512, 1024, 2048, 6000):
+        with tuning("mfma_min_chunk", stated):
+            for target in (0, 64):
+                work, nu, nr = ops.decode_plan(lens, 14, 2, D, 16, target_tokens=target)
+                chunks = np.bincount(work[:, 0]) // 2
+                assert (chunks[lens <= stated] == 1).all() and chunks[0] > 1
+                whole = work[:, 4] & 0xFFFF == 1
+                assert (work[~whole, 3] - work[~whole, 2]).max() >= stated * 2 // 3
+    assert lib().kvc_set_tuning(b"mfma_min_chunk", 8) != 0
