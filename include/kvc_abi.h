@@ -266,7 +266,10 @@ int kvc_decode_auto_split(int N, int Hq, int Hkv, int D, int BLOCK, int cap, int
  * matrix-core path (64-int entries) by up to 56 of the chunk's block ids copied
  * from host_table_all (may be NULL: then none are inlined).  host_tab_off (N+1,
  * may be NULL: tables packed in sequence order) locates each sequence's table in
- * table_all.  target_tokens = 0 picks the chunk size.  capacity is in units.  The
+ * table_all.  target_tokens = 0 picks the chunk size; a smaller request than the batch's
+ * least chunk is raised to it (grouped-query heads on the matrix cores: 1024 tokens where
+ * that splits nothing, else a twelfth of the longest sequence within 256..1024, or
+ * "mfma_min_chunk").  capacity is in units.  The
  * caller copies the work list to the device (e.g. inside its per-step upload) and
  * runs kvc_batched_paged_decode_planned with the same shape and tables; every
  * block-id read is bounded by table_len (ints in table_all).  Partials of split

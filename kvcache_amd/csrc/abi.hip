@@ -392,12 +392,13 @@ constexpr int kPlanIntsInline = 64;   // grouped-query units: header + up to 56 
 
 struct PlanShape {
     int G, nsub, hks, tpw, wpb, min_chunk, max_chunk, slots, entry_ints;
-    int min_chunk_long = 0;  // mfma: min_chunk for batches with long sequences (plan_min_chunk)
+    int coarse = 0, fine = 0;  // mfma: gqa_chunk_target's least chunks
+    int wide_chunk = 0;        // mfma: largest automatic target of uneven batches, 0: none
     int target_cap = INT_MAX;  // largest automatic chunk target (tokens)
     bool uniform, mfma;
 };
 
-// N: sequences of the launch (waves per unit only; the units do not depend on it).
+// N: sequences of the launch (waves per unit, and with them the largest target).
 PlanShape plan_shape(int Hq, int Hkv, int D, int BLOCK, int dtype, int N = 0) {
     PlanShape ps{};
     const int group = Hq / Hkv;
@@ -411,28 +412,25 @@ PlanShape plan_shape(int Hq, int Hkv, int D, int BLOCK, int dtype, int N = 0) {
         ps.tpw = 32;
         // head_dim 128: 4 waves (8 spill 41-125 registers and leave no CU a second unit:
         // 200 sequences of 32..4096 tokens, 32q/8kv, planned 209 -> 131 us, 16 sequences
-        // 28.3 -> 21.9).  head_dim 64: 8, and 4 once the units fill the chip several times
-        // (units of 64 lengths 14.8 us at 8 waves, 18.5 at 4; 500 x 2 19.8 and 15.9)
+        // 28.3 -> 21.9), but for a few units of more than 8 heads, whose merge is the tail
+        // (16q/1kv, one sequence of 32768: 41.4 us at 4 waves, 33.7 at 8; 8 of them 44 and
+        // 46).  head_dim 64: 8, and 4 once the units fill the chip several times (units of
+        // 64 lengths 14.8 us at 8 waves, 18.5 at 4; 500 x 2 19.8 and 15.9)
         const int t = tuning().waves_per_block;
-        ps.wpb = (t == 4 || t == 8) ? t : (D == 128 || (long long)N * Hkv >= 768 ? 4 : 8);
-        // a split costs the chunk tail a store, an arrival and a merge: sequences stay whole
-        // up to 1.5 chunks of at least min_chunk_long tokens, an eighth of the longest
-        // sequence between 512 (64 sequences of 128..4096 tokens 14.8 -> 13.6 us) and 1024
-        // (4 of 8192..32768: 15.3 us, 17.8 in chunks of 704), or min_chunk_long where that
-        // splits nothing (12 layers, 7 sequences x 4 KV heads of at most 1000 tokens: 83 us
-        // whole, 120 in chunks of at least 512: a merge for no chunk after it) and once whole
-        // sequences fill the CUs (60 sequences x 8 KV heads, D 128: 23.8 us, 27.0 in chunks
-        // of at least 512; 128 x 4, D 64: 15.1 and 16.1)
+        const long long pairs = (long long)N * Hkv;
+        ps.wpb = (t == 4 || t == 8) ? t
+               : D == 128           ? (group > 8 && pairs < 8 ? 8 : 4)
+                                    : (pairs >= kGqaWidePairs ? 4 : 8);
+        // a split costs the chunk tail a store, an arrival and a merge (gqa_chunk_target); a
+        // stated mfma_min_chunk is the least chunk of every batch
         auto blocks_up = [&](int x) { return (x + BLOCK - 1) / BLOCK * BLOCK; };
-        // a stated mfma_min_chunk is the least chunk of every batch
         const int stated = tuning().mfma_min_chunk;
-        ps.min_chunk = blocks_up(stated > 0 ? stated : 512);
-        ps.min_chunk_long = blocks_up(stated > 0 ? stated : 1024);
+        ps.coarse = blocks_up(stated > 0 ? stated : 1024);
+        ps.fine = stated > 0 ? 0 : blocks_up(256);
+        ps.min_chunk = stated > 0 ? ps.coarse : ps.fine;
+        ps.wide_chunk = D == 64 && pairs >= kGqaWidePairs && stated == 0 ? blocks_up(kGqaWideChunk) : 0;
         ps.max_chunk = kMfmaMaxChunkBlocksHost * BLOCK;
-        // units to aim for: one per CU for head_dim 64; for 128 about two, whose shorter
-        // chunks balance the rounds of a large batch (200 sequences, device lengths: 172
-        // us aiming at 176 units, 160 at 256, 148 at 512)
-        ps.slots = D == 128 ? 512 : 256;
+        ps.slots = kGqaSlots;
         // the unit's first block ids travel in its entry: the kernel reads entry and
         // ids in one round instead of entry, then table
         ps.entry_ints = kPlanIntsInline;
@@ -469,41 +467,37 @@ inline int plan_key(bool split, long long len, int T, bool split_first) {
     return (split && split_first ? 64 : 0) + b;
 }
 
+// The chunk target (tokens) of a plan: `target`, or automatically enough units to
+// fill the machine's slots about once, at least min_chunk, a multiple of BLOCK.
+int plan_chunk_target(const int* lens, int N, const PlanShape& ps, int BLOCK, int target) {
+    long long tokens = 0;
+    int lmax = 0;
+    for (int i = 0; i < N; ++i) {
+        tokens += std::max(lens[i], 1);
+        lmax = std::max(lmax, lens[i]);
+    }
+    auto over = [&](int slots) {
+        return (int)std::min<long long>((tokens * ps.hks + slots - 1) / slots, INT_MAX / 2);
+    };
+    const bool automatic = target <= 0;
+    int T = automatic ? std::min(over(ps.slots), ps.target_cap) : target;
+    if (ps.mfma) {
+        T = gqa_chunk_target(std::min(T, INT_MAX / 2), automatic ? over(kGqaSplitSlots) : T, lmax, ps.coarse, ps.fine, BLOCK);
+        if (automatic && ps.wide_chunk && (long long)lmax * N > 2 * tokens) T = std::min(T, ps.wide_chunk);
+    } else {
+        T = std::max(T, ps.min_chunk);
+        T = (T + BLOCK - 1) / BLOCK * BLOCK;
+    }
+    return std::min(T, ps.max_chunk);
+}
+
 // Two passes, no sort: the first cuts every sequence into chunks and counts the
 // units per order key (all a size query needs), the second writes each unit at its
 // key's next slot (a counting sort; within a key in generation order: sequence, then
 // chunks 0..nc-2 of every head, then the last chunk of every head).
-// The chunk target (tokens) of a plan: `target`, or automatically enough units to
-// fill the machine's slots about once, at least min_chunk, a multiple of BLOCK.
-// Least automatic or requested chunk for a batch of N sequences whose longest has lmax
-// tokens (the kernel's own planner applies the same rule).
-int plan_min_chunk(const PlanShape& ps, int N, int lmax, int BLOCK) {
-    if (!ps.mfma) return ps.min_chunk;
-    if ((long long)N * ps.hks >= kPlanFullUnits || lmax <= plan_whole_max(ps.min_chunk_long))
-        return std::max(ps.min_chunk, ps.min_chunk_long);
-    const int eighth = (int)std::min<long long>(((long long)lmax / 8 + BLOCK - 1) / BLOCK * BLOCK, ps.min_chunk_long);
-    return std::max(ps.min_chunk, eighth);
-}
-
-int plan_chunk_target(const int* lens, int N, const PlanShape& ps, int BLOCK, int target) {
-    long long total = 0;
-    int lmax = 0;
-    for (int i = 0; i < N; ++i) {
-        total += std::max(lens[i], 1);
-        lmax = std::max(lmax, lens[i]);
-    }
-    total *= ps.hks;
-    if (target <= 0)
-        target = (int)std::min<long long>(std::min<long long>((total + ps.slots - 1) / ps.slots, ps.target_cap),
-                                          INT_MAX / 2);
-    int T = std::max(target, plan_min_chunk(ps, N, lmax, BLOCK));
-    T = (T + BLOCK - 1) / BLOCK * BLOCK;
-    return std::min(T, ps.max_chunk);
-}
-
 int make_plan(const int* lens, const int* tab_off, const int* table, int table_len, int N, int Hq, int Hkv, int D,
               int BLOCK, int dtype, int target, int* work, int capacity, int* n_units, int* n_records) {
-    const PlanShape ps = plan_shape(Hq, Hkv, D, BLOCK, dtype);
+    const PlanShape ps = plan_shape(Hq, Hkv, D, BLOCK, dtype, N);
     if (ps.hks > 0xFFFF) return set_error(KVC_ERR_UNSUPPORTED, "too many KV heads for the plan encoding");
     const int T = plan_chunk_target(lens, N, ps, BLOCK, target);
     const bool split_first = tuning().split_first != 0;
@@ -861,7 +855,8 @@ int run_self_planned(const void* q, const void* k, const void* v, const int* tab
     p.n_records = (int)recs;
     p.lpb_shift = ilog2_exact(BLOCK / ps.tpw);  // uniform paging (self_plan_ok)
     p.sp_slots = ps.slots; p.sp_min_chunk = ps.min_chunk; p.sp_max_chunk = ps.max_chunk;
-    p.sp_min_long = ps.min_chunk_long;
+    if (ps.mfma) p.sp_min_chunk = ps.coarse;
+    p.sp_fine_chunk = ps.fine; p.sp_wide_chunk = ps.wide_chunk;
     p.sp_target_cap = ps.target_cap; p.sp_nc_max = ps.mfma ? kMfmaMaxFusedChunks : 0;
     p.sp_records = self_plan_budget(ps, bound);
     if (!contig && cur_len && tab_off && tuning().self_prefetch_kib > 0) {
@@ -1442,7 +1437,7 @@ int kvc_decode_plan_chunk(const int* host_lens, int N, int Hq, int Hkv, int D, i
         if (N < 0 || (N > 0 && !host_lens) || Hq <= 0 || Hkv <= 0 || Hq % Hkv || BLOCK <= 0 || !d_ok(D) ||
             !dtype_ok(dtype))
             return set_error(KVC_ERR_ARG, "bad plan arguments");
-        *chunk_tokens = kvc::plan_chunk_target(host_lens, N, kvc::plan_shape(Hq, Hkv, D, BLOCK, dtype), BLOCK,
+        *chunk_tokens = kvc::plan_chunk_target(host_lens, N, kvc::plan_shape(Hq, Hkv, D, BLOCK, dtype, N), BLOCK,
                                                target_tokens);
         return KVC_OK;
     });

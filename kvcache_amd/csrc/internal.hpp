@@ -77,7 +77,8 @@ struct DecodeParams {
     // queries whose first position lives in device memory, that position (query s
     // then attends to *dev_base + s + 1 keys; causal must be 1)
     int sp_slots, sp_min_chunk, sp_max_chunk, sp_target_cap;
-    int sp_min_long;          // matrix cores: sp_min_chunk of batches with long sequences (plan_min_chunk), else 0
+    int sp_fine_chunk;        // matrix cores: gqa_chunk_target's fine (sp_min_chunk: its coarse)
+    int sp_wide_chunk;        // matrix cores: largest target of uneven batches (kGqaWideChunk), 0: none
     int sp_nc_max;            // chunks per sequence the merge can combine (0: any)
     int sp_records;           // partial records per (sequence, head) in the workspace
     int sp_pf_blocks;         // blocks of every sequence read ahead while the plan is made (0: none)
@@ -110,12 +111,36 @@ int* device_error_word(hipStream_t st, bool may_alloc);
 bool take_device_error_code(int code);
 int device_error_status(int code);
 
-// Grouped-query decode: with this many (sequence, KV head) pairs, one per CU, sequences are
-// only split into long chunks (plan_min_chunk).
-constexpr int kPlanFullUnits = 256;
-// ... and a batch with no longer sequence than this stays whole in chunks of at least
-// `chunk` (split_seq's rule: up to 1.5 chunks).
-constexpr long long plan_whole_max(int chunk) { return (long long)chunk * 3 / 2; }
+// Chunk target of a grouped-query batch, for the host planner and the kernel's own (the same
+// chunks bit for bit).  t: the tokens of every KV head over kGqaSlots units (or a requested
+// target), ts: over kGqaSplitSlots, lmax: the longest sequence, coarse: the least chunk of a
+// batch that stays whole, fine: of one that is split anyway (0: coarse is a stated minimum).
+//
+// Chunks of about 0.7 of a unit per CU (kGqaSlots) keep a large batch of equal sequences in
+// one round, and one that this splits nothing of pays for no merge: 128 sequences of 1700
+// tokens, 16q/1kv, D 64, 14.7 us whole, 19.1 cut for 256 units; 3 of 32768, 64q/8kv, 36.5 us
+// in 168 units, 49.7 in 264.  Where the longest sequence is split at `coarse` all the same, and
+// the batch is small, finer chunks shorten its chain and their merges run beside each other: a
+// twelfth of the longest, up to kGqaSplitSlots units.  64 sequences of 32..4096 tokens, 14q/2kv:
+// 13.9 us at 1024, 11.2 at 608; 5 sequences 11.5 and 10.3; one of 4096, 32q/8kv, D 128: 18.9
+// and 13.7; over 900 batches of 1 to 300 sequences no case above 1.08 of one chunk rule for
+// all (1024), D 64 0.96 and D 128 0.75 of its time on average.
+constexpr int kGqaSlots = 176, kGqaSplitSlots = 240;
+__host__ __device__ inline int gqa_chunk_target(int t, int ts, int lmax, int coarse, int fine, int block) {
+    auto blocks_up = [&](int x) { return (x + block - 1) & ~(block - 1); };
+    const int T = blocks_up(t > coarse ? t : coarse);
+    if (fine == 0 || t > coarse || lmax <= T + T / 2) return T;
+    int least = lmax / 12;
+    least = least > fine ? least : fine;
+    least = least < coarse ? least : coarse;
+    return blocks_up(ts > least ? ts : least);
+}
+
+// ... and the largest target of units of four waves (head_dim 64, kGqaWidePairs and more): a
+// sequence far above the mean is the batch's tail there (128 sequences of 32..4096 tokens,
+// 32q/8kv, 45.0 us whole, 38.2 with its long ones in two; 39.5 with eight waves).  Not for
+// equal lengths (128 of 4096: 186 us whole, 197 in two).
+constexpr int kGqaWidePairs = 768, kGqaWideChunk = 2048;
 
 // Prompt attention at a device position with fewer keys than this is never split over
 // workgroups: up to here one workgroup's key streams take about as long as a split's partials

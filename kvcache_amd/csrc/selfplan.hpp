@@ -222,14 +222,15 @@ __device__ SelfPlan self_plan_setup(const int* lens, int n_seq, const DecodePara
         else if (pmax <= 0xFFFFFFFFull) c = ceil_div_u32((unsigned)prod, (unsigned)p.sp_slots);
         else c = ceil_div_u64((long long)prod, p.sp_slots);
         long long T = min(c, (long long)p.sp_target_cap);
-        long long least = p.sp_min_chunk;
-        if constexpr (!Lds::kLead) {  // matrix cores: plan_min_chunk's rule
-            const bool whole = (long long)N * hks >= kPlanFullUnits || lall <= plan_whole_max(p.sp_min_long);
-            const long long eighth = whole ? (long long)p.sp_min_long : (((long long)lall >> 3) + B - 1) >> bsh << bsh;
-            least = max(least, min(eighth, (long long)p.sp_min_long));
+        if constexpr (Lds::kLead) {
+            T = max(T, (long long)p.sp_min_chunk);
+            T = (T + B - 1) >> bsh << bsh;
+        } else {  // matrix cores (prod fits 32 bits where ts is used: t is at most coarse there)
+            T = gqa_chunk_target((int)T, (int)ceil_div_u32((unsigned)prod, kGqaSplitSlots), lall, p.sp_min_chunk,
+                                 p.sp_fine_chunk, B);
+            if (p.sp_wide_chunk && (unsigned long long)(unsigned)lall * (unsigned)N > 2 * tokens)
+                T = min(T, (long long)p.sp_wide_chunk);
         }
-        T = max(T, least);
-        T = (T + B - 1) >> bsh << bsh;
         T = min(T, (long long)M);
         // ... raised to the record budget (and the 64-chunk merge of the matrix-core
         // path): fit = ceil(tokens / ((sp_records - 1) * N)); past M only that matters

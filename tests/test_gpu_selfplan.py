@@ -394,16 +394,20 @@ def test_block_table_at_the_end_of_its_allocation(orc, n, causal):
     assert np.abs(got - ref).max() <= 2e-3
 
 
-@pytest.mark.parametrize("D,Hq,Hkv,n", [(64, 14, 2, 3), (64, 28, 4, 70), (64, 32, 8, 96), (128, 8, 2, 5),
-                                        (128, 32, 8, 33)])
-def test_grouped_units_host_and_device_plans(orc, D, Hq, Hkv, n):
-    # the grouped-query units' rules on the batch: fewer (sequence, KV head) pairs than
-    # kPlanFullUnits (chunks from an eighth of the longest sequence), at least that many,
-    # and at least 768 (4 waves at D 64); device lengths and host plan agree bit for bit
+# wide: sequences far above the mean among 768 (sequence, KV head) pairs
+@pytest.mark.parametrize("D,Hq,Hkv,n,wide", [(64, 14, 2, 3, 0), (64, 28, 4, 70, 0), (64, 32, 8, 96, 0), (64, 32, 8, 96, 1),
+                                             (128, 8, 2, 5, 0), (128, 32, 8, 33, 0), (128, 16, 1, 7, 0),
+                                             (128, 16, 1, 9, 0)])
+def test_grouped_units_host_and_device_plans(orc, D, Hq, Hkv, n, wide):
+    # the grouped-query units' rules on the batch (gqa_chunk_target): chunks of a twelfth of the
+    # longest sequence, of a 176th of the batch, the largest target of four-wave units, and the
+    # waves per unit; device lengths and host plan agree bit for bit
     say(f"grouped units D={D} Hq={Hq} Hkv={Hkv} n={n}")
     rng = np.random.default_rng(n)
     lens = rng.integers(1, 400, n).astype(np.int32)
     lens[:3] = (4200, 1549, 900)
+    if wide:
+        lens[4::8] = 3500
     B = 16
     nb = int(sum((int(x) + B - 1) // B for x in lens))
     alloc = BlockAllocator(nb)
@@ -425,8 +429,8 @@ def test_grouped_units_host_and_device_plans(orc, D, Hq, Hkv, n):
 @pytest.mark.parametrize("D,Hq,Hkv", [(64, 28, 4), (128, 8, 2)])
 @pytest.mark.parametrize("longest", [1000, 1536, 1537])
 def test_short_grouped_batches_stay_whole(orc, D, Hq, Hkv, longest):
-    # up to one and a half of the long chunks nothing is split (a split's merge costs more
-    # than it saves); both planners draw the line at the same length
+    # up to one and a half chunks of 1024 nothing is split (a split's merge costs more than it
+    # saves); both planners draw the line at the same length
     say(f"short grouped batch D={D} longest={longest}")
     lens = np.array([longest, 800, 33, 1, 700], np.int32)
     n, B = len(lens), 16

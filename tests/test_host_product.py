@@ -372,3 +372,28 @@ def test_stated_min_chunk_keeps_shorter_sequences_whole(D):
                 whole = work[:, 4] & 0xFFFF == 1
                 assert (work[~whole, 3] - work[~whole, 2]).max() >= stated * 2 // 3
     assert lib().kvc_set_tuning(b"mfma_min_chunk", 8) != 0
+
+
+def test_grouped_plans_split_only_what_gains():
+    # equal sequences that the units' number alone would split stay whole (a merge for nothing),
+    # the units of a few long ones stay within one round of the 256 CUs, and a batch whose
+    # longest sequence is split anyway is cut finer
+    from kvcache_amd import ops
+
+    def plan(lens, Hq, Hkv, D):
+        work, nu, nr = ops.decode_plan(np.asarray(lens, np.int32), Hq, Hkv, D, 16)
+        return nu, nr, int((work[:, 3] - work[:, 2]).max())
+
+    for D in (64, 128):
+        for n, Hq, Hkv, L in ((128, 16, 1, 1700), (32, 28, 4, 2500), (16, 64, 8, 4096), (64, 14, 2, 1700)):
+            assert plan([L] * n, Hq, Hkv, D)[:2] == (n * Hkv, 0)
+        for n, Hq, Hkv in ((3, 64, 8), (5, 14, 2), (5, 28, 4)):
+            assert plan([32768] * n, Hq, Hkv, D)[0] <= 192
+        lens = W.loguniform_lengths(64, 32, 4096, 5)
+        nu, nr, longest = plan(lens, 14, 2, D)
+        assert nr > 0 and longest <= 900
+        assert plan([4096], 32, 8, D)[2] <= 384
+    # four waves per unit (768 pairs and more, D 64): sequences far above the mean are split
+    lens = [3500] * 12 + [200] * 84
+    assert plan(lens, 32, 8, 64)[2] <= 2048 and plan(lens, 32, 8, 128)[2] == 3500
+    assert plan([4096] * 128, 32, 8, 64)[:2] == (1024, 0)
