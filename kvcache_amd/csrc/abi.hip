@@ -70,6 +70,7 @@ int choose_g(int group, int D) {
 // hold whole 16-token subtiles.
 constexpr int kMfmaMaxChunkBlocksHost = 1024;
 constexpr int kMfmaMaxFusedChunks = 64;
+constexpr int kAutoFusedChunks = 8;  // grids of chunks: more are merged by merge_kernel
 inline bool mfma_path(int group, int D, int dtype, int BLOCK, bool paged) {
     const int t = tuning().mfma;
     if (t == 0 || dtype != KVC_F16 || (D != 64 && D != 128) || group > 16 || group < (t == 1 ? 3 : 4)) return false;
@@ -132,7 +133,7 @@ void size_workspace(Plan& pl, int N, int Hq, int Hkv, int D) {
     pl.ws_bytes = pl.acc_bytes + pl.ml_bytes + align_up(ctr_region_bytes(pl.n_ctr), kAlign);
 }
 
-// Matrix-core path: all heads of the group per unit, 8 waves per unit, chunks of
+// Matrix-core path: all heads of the group per unit, 4 or 8 waves per unit, chunks of
 // at least two 32-token tiles per wave, about 512 units over the longest length.
 Plan plan_batched_mfma(int N, int Hq, int Hkv, int D, int BLOCK, int cap, int split, bool paged) {
     Plan pl;
@@ -151,10 +152,18 @@ Plan plan_batched_mfma(int N, int Hq, int Hkv, int D, int BLOCK, int cap, int sp
     if (paged && ch % BLOCK) ch = (ch + BLOCK - 1) / BLOCK * BLOCK;
     pl.chunk = (int)std::min<long long>(ch, 1 << 24);
     pl.max_chunks = std::max(1, (std::max(cap, 0) + pl.chunk - 1) / pl.chunk);
-    // 4 waves per unit once there are enough units to fill the CUs (head_dim 128: always,
-    // as plan_shape), else 8
+    // 4 waves per unit once there are enough units to fill the CUs, else 8.  head_dim 128: 4
+    // always (8 spill: 192 units of 512 tokens, 32q/8kv, 21.5 -> 17.8 us), but for a few
+    // units of 8 heads or more whose merge in the launch is the tail (up to 8 chunks, then
+    // merge_kernel; chunks of 512, 16q/1kv: 2 units 21.0 us at 8 waves, 25.5 at 4, 96 units
+    // 22.7 and 26.0, 128 units of 16 chunks 19.6 and 15.7; 32q/4kv: 16 units 16.0 and 17.3, 128
+    // units 19.0 and 17.9)
     const int t = tuning().waves_per_block;
-    pl.wpb = (t == 4 || t == 8) ? t : (D == 128 || (long long)pl.max_chunks * N * Hkv >= 256 ? 4 : 8);
+    const long long units = (long long)pl.max_chunks * N * Hkv;
+    const bool merges = pl.max_chunks > 1 && pl.max_chunks <= kAutoFusedChunks;
+    pl.wpb = (t == 4 || t == 8) ? t
+           : D == 128           ? (pl.G >= 8 && merges && units < 128 ? 8 : 4)
+                                : (units >= 256 ? 4 : 8);
     pl.mode = paged ? kPagedUniform : kContiguous;
     pl.chunk_blocks_ok = !paged || pl.chunk / BLOCK <= kMfmaMaxChunkBlocksHost;
     size_workspace(pl, N, Hq, Hkv, D);
@@ -324,7 +333,7 @@ int resolve_workspace(const Plan& pl, void* ws, size_t ws_bytes, DecodeParams& p
     p.ctr_shift = ctr_shift_for(pl.n_ctr);
     p.epoch = next_epoch();
     const int t = tuning().fused_merge;
-    p.merge_mode = t >= 0 ? t : (pl.max_chunks <= 8 ? kMergeAtomic : kMergeKernel);
+    p.merge_mode = t >= 0 ? t : (pl.max_chunks <= kAutoFusedChunks ? kMergeAtomic : kMergeKernel);
     // the matrix-core kernel's fused merge holds one chunk per lane
     if (pl.mfma && pl.max_chunks > kMfmaMaxFusedChunks) p.merge_mode = kMergeKernel;
     return KVC_OK;

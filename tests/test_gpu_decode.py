@@ -455,6 +455,20 @@ def test_mfma_merge_modes(orc, mode):
             assert np.abs(got - ref).max() <= 2e-3
 
 
+# stated splits at head_dim 128: four waves, and eight for up to 127 units of 8 heads or more
+# that are merged in the launch (2 to 8 chunks)
+@pytest.mark.parametrize("Hq,Hkv,longest,split", [(16, 1, 500, 512), (16, 1, 1100, 512), (16, 1, 4700, 512),
+                                                  (32, 4, 1100, 512), (8, 2, 1100, 512), (32, 4, 4000, 128)])
+def test_mfma_d128_stated_splits(orc, Hq, Hkv, longest, split):
+    say(f"mfma D 128 stated split Hq={Hq} Hkv={Hkv} longest={longest} split={split}")
+    lens = np.array([longest, longest // 3, 17], np.int32)
+    N, D = len(lens), 128
+    q, K, V = (normal((N, h, longest, D) if h is not None else (N, Hq, D), 190 + i, np.float16)
+               for i, h in enumerate((None, Hkv, Hkv)))
+    got = run_batched(q, K, V, lens, Hkv, 16, KVC_F16, split=split)
+    assert np.abs(got - oracle_out(orc, q, K, V, lens)).max() <= tol(KVC_F16)
+
+
 # ---- prompt (prefill) attention: qk_paged_causal_attn (qwen_kernels.h:19-21) ---------
 @pytest.mark.parametrize("dtype,Hq,Hkv", [(KVC_F16, 14, 2), (KVC_F16, 8, 8), (KVC_F32, 8, 2)])
 @pytest.mark.parametrize("base,n", [(0, 1), (0, 37), (100, 64), (0, 600), (5000, 3)])
