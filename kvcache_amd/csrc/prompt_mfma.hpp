@@ -9,10 +9,15 @@
 //   QK^T  : S^T[32 keys][32 queries] = K Q^T with v_mfma_f32_32x32x16_f16, so a lane
 //           holds 16 scores of ONE query (column l % 32): the row maximum and sum need one
 //           exchange with lane l ^ 32, and the rescale factor is a per-lane scalar.
-//   softmax: fp32 online (max, sum, acc) in log2 units; O is rescaled only when some
-//           query of the wave met a new maximum.  (Letting the maximum lag behind by up to
-//           2^8 saved most rescales, but its error against 64 bits was 3% larger: fewer
-//           probabilities are exactly 1.)
+//   softmax: fp32 online (reference, sum, acc) in log2 units; O is rescaled only when some
+//           query of the wave met a new maximum.  head_dim 128: then every query takes the
+//           tile's own maximum as its reference (at most 2^8 below its running maximum), since
+//           a probability of exactly 1 loses nothing to its rounding to fp16, and the fewer
+//           maxima the key streams have between them, the larger the error (1000 queries
+//           behind 6000 keys, against 64 bits: running maxima of two streams 2.83e-4, of the
+//           four of the 16-query units before 2.80e-4, this 2.69e-4; 100 behind 1500 2.66e-4,
+//           2.61e-4, 2.53e-4).  At head_dim 64 running maxima are no further off than those
+//           units were (2.45e-4 and 2.47e-4 at 2048 queries), and this cost 3% there.
 //   PV    : O^T[32 dims][32 queries] += V^T P^T.  The lane's own probabilities are in the
 //           B operand layout up to the order of the keys, and V^T is read back in that
 //           order with the transposing LDS read, so P never leaves its registers.
@@ -185,6 +190,7 @@ __global__ __launch_bounds__(W * kWave) void prompt_kernel(DecodeParams p) {
         for (int d = 0; d < KD; ++d) qb[d] = -qb[d];
     }
     float m = -FLT_MAX, l = 0.f;  // of this column; l of the lane's own keys only
+    float top = -FLT_MAX;         // its running maximum (m: the reference of l and O; D 64: both)
     f32x16 O[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -217,8 +223,8 @@ __global__ __launch_bounds__(W * kWave) void prompt_kernel(DecodeParams p) {
         }
         // S[n][i] is key t0 + 32 n + 8 (i / 4) + 4 h + i % 4
         const int lim = qlast - t0 - 4 * h;  // seen when 32 n + 8 (i / 4) + i % 4 <= lim
-        // each 32-key subtile against its own running maximum (over 64 keys at a time the
-        // error against 64 bits was 1% larger: fewer probabilities are exactly 1)
+        // each 32-key subtile against its own maximum (over 64 keys at a time the error
+        // against 64 bits was 1% larger: fewer probabilities are exactly 1)
 #pragma unroll
         for (int n = 0; n < NS; ++n) {
             auto seen = [&](int i) { return !MASKED || 32 * n + 8 * (i >> 2) + (i & 3) <= lim; };
@@ -226,8 +232,9 @@ __global__ __launch_bounds__(W * kWave) void prompt_kernel(DecodeParams p) {
 #pragma unroll
             for (int i = 0; i < 16; ++i) mx = seen(i) ? fmaxf(mx, S[n][i]) : mx;
             mx = max_xor32(mx) * sl2;
-            if (__any(mx > m)) {
-                const float mn = fmaxf(m, mx);
+            if (__any(mx > (D == 128 ? top : m))) {
+                if constexpr (D == 128) top = fmaxf(top, mx);
+                const float mn = D == 128 ? fmaxf(mx, top - 8.f) : fmaxf(m, mx);
                 const float corr = fast_exp2(m - mn);
                 m = mn;
                 l *= corr;
@@ -451,11 +458,11 @@ __global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kern
 #pragma unroll
             for (int d = 0; d < KD; ++d) qb[n][d] = -qb[n][d];
     }
-    float m[NC], l[NC];
+    float m[NC], l[NC], top[NC];  // as prompt_kernel's
     f32x16 O[NC][DT];
 #pragma unroll
     for (int n = 0; n < NC; ++n) {
-        m[n] = -FLT_MAX;
+        m[n] = top[n] = -FLT_MAX;
         l[n] = 0.f;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
@@ -491,8 +498,9 @@ __global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kern
 #pragma unroll
             for (int i = 0; i < 16; ++i) mx = seen(i) ? fmaxf(mx, S[n][i]) : mx;
             mx = max_xor32(mx) * sl2;
-            if (__any(mx > m[n])) {
-                const float mn = fmaxf(m[n], mx);
+            if (__any(mx > (D == 128 ? top[n] : m[n]))) {
+                if constexpr (D == 128) top[n] = fmaxf(top[n], mx);
+                const float mn = D == 128 ? fmaxf(mx, top[n] - 8.f) : fmaxf(m[n], mx);
                 const float corr = fast_exp2(m[n] - mn);
                 m[n] = mn;
                 l[n] *= corr;
@@ -526,7 +534,8 @@ __global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kern
         __builtin_amdgcn_wave_barrier();
         stage();
         if constexpr (decltype(masked_tag)::value) {  // (while the LDS writes are under way)
-            if (any_nonfinite(rv[0]) | any_nonfinite(rv[1])) {
+            const bool bad0 = any_nonfinite(rv[0]), bad1 = any_nonfinite(rv[1]);
+            if (bad0 || bad1) {
                 clear_nonfinite(rv[0]);
                 clear_nonfinite(rv[1]);
                 bad = true;

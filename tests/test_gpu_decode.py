@@ -586,6 +586,41 @@ def test_device_position_keeps_probabilities_in_32_bits(orc, D, Hq, Hkv, n):
     assert np.mean(got != want.astype(np.float16)) <= 0.02
 
 
+@pytest.mark.parametrize("case,bound", [("tiles", 2.763e-4), ("streams", 2.517e-4), ("units", 2.630e-4)])
+def test_head_dim_128_error_against_64_bits(orc, case, bound):
+    """The fp16 rounding of the probabilities costs no more than it did with 16 queries per unit
+    and eight waves per decode unit: the bounds are the 2-norm errors of those kernels on these
+    inputs.  128-query tiles with the running maxima of two key streams gave 2.794e-4,
+    32-query tiles of eight streams 2.603e-4, four-wave decode units 2.681e-4; the tiles' own
+    maxima 2.661e-4, 2.491e-4 and 2.512e-4 (the output's own rounding is 2.04e-4 of each)."""
+    say(f"error against 64 bits D=128 {case}")
+    D, B, Hkv = 128, 16, 2
+    Hq, base, n = {"tiles": (40, 6000, 520), "streams": (8, 1500, 100), "units": (16, 1448, 1)}[case]
+    nb = (base + n + B - 1) // B
+    table = np.random.default_rng(5).permutation(nb).astype(np.int32)
+    kp, vp = normal((nb, Hkv, B, D), 240, np.float16), normal((nb, Hkv, B, D), 241, np.float16)
+    scale = float(1.0 / np.sqrt(D))
+    q = normal((n, Hq, D), 242, np.float16)
+    if case == "units":  # 40 sequences over the one table
+        n = 40
+        q = normal((n, Hq, D), 242, np.float16)
+        out = DeviceBuffer(q.nbytes)
+        lens = np.full(n, base, np.int32)
+        ops.launch_batched_paged(dev(q), dev(kp), dev(vp), dev(table), dev(np.zeros(n + 1, np.int32)), dev(lens), out, n,
+                                 Hq, D, B, base, scale, Hkv=Hkv, dtype=KVC_F16)
+        want = orc.batched_paged(q, kp, vp, table, np.zeros(n + 1, np.int32), lens, Hkv, B, scale, nthreads=8)
+    else:
+        out = DeviceBuffer(q.nbytes)
+        ops.qk_paged_causal_attn(dev(q), out, dev(kp), dev(vp), dev(table), base, n, Hq, Hkv, D, B, scale)
+        rows = np.arange(0, n, 13)  # (some queries: the oracle takes a second per hundred)
+        want = orc.batched_paged(q[rows], kp, vp, table, np.zeros(len(rows) + 1, np.int32),
+                                 (base + 1 + rows).astype(np.int32), Hkv, B, scale, nthreads=8)
+    got = host(out, np.float16, q.shape).astype(np.float64)
+    if case != "units":
+        got = got[rows]
+    assert np.linalg.norm(got - want) / np.linalg.norm(want) <= bound
+
+
 def test_prefill_flow_write_then_causal_attn(orc):
     """The model path's prefill (qwen_serve.cu:106-108): write the P prompt rows of
     K/V through the sequence's table, then causal attention over them."""
