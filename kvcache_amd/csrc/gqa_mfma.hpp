@@ -232,8 +232,10 @@ __global__ __launch_bounds__(WPB * kWave) void gqa_mfma_kernel(const int* __rest
     // 16-byte chunk of a K row in LDS: the sixteen rows one operand read touches
     // (same chunk) spread over the banks
     auto kchunk = [](int r, int c) { return c ^ (r & 7); };
-    // per head n16 (identical in the four lane groups): running maximum, reference of l and O
-    float top = -FLT_MAX, m = -FLT_MAX, l = 0.f;
+    // per head n16 (identical in the four lane groups): reference of l and O; running maximum
+    // where that is not it
+    float m = -FLT_MAX, l = 0.f;
+    [[maybe_unused]] float top = -FLT_MAX;
     f32x4 O[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) O[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -283,12 +285,16 @@ __global__ __launch_bounds__(WPB * kWave) void gqa_mfma_kernel(const int* __rest
             mx = ok[i] ? fmaxf(mx, S[h][r]) : mx;
         }
         mx = max_xor32(max_xor16(mx));
-        // the tile's own maximum is its reference (at most 2^16 below the running one): O is
-        // rescaled for every tile anyway, and a probability of exactly 1 loses nothing to its
-        // rounding to fp16 (200 sequences, 32q/8kv, D 128, four waves: error against 64 bits
-        // 2.56e-4 with running maxima, with eight waves 2.55e-4, so 2.4e-4)
-        top = fmaxf(top, mx * sl2);
-        const float mn = fmaxf(mx * sl2, top - 16.f);
+        // Four waves have half the running maxima of eight, and a probability of exactly 1
+        // loses nothing to its rounding to fp16 (200 sequences, 32q/8kv, D 128, error against
+        // 64 bits: 2.549e-4 with eight waves, 2.559e-4 with four).  O is rescaled for every
+        // tile anyway, so the tile's own maximum is its reference, at most 2^16 below the
+        // running one: at head_dim 128 of every tile (2.541e-4), at 64 of every second tile of
+        // four waves (128 sequences, 32q/8kv: 2.544e-4 with eight, 2.555e-4, so 2.546e-4); eight
+        // waves there keep the running maximum
+        constexpr bool kOwn = D == 128, kSecond = D == 64 && WPB == 4;
+        if constexpr (kOwn || kSecond) top = fmaxf(top, mx * sl2);
+        const float mn = kOwn || (kSecond && (k & 1) == 0) ? fmaxf(mx * sl2, top - 16.f) : fmaxf(m, mx * sl2);
         const float corr = fast_exp2(m - mn);
         float ps = 0.f;
         f16x8v pa;
