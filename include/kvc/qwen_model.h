@@ -12,9 +12,9 @@
 // K/V written in the same launch; output projection + residual; RMSNorm + gate/up
 // projection + SwiGLU; down projection + residual; then final norm + lm_head +
 // argmax.  Prompts and larger batches run RMSNorm and the fused linear layers of many rows
-// (kvc_block_qkv / swiglu / linear), with the prompts' K/V stored by the q/k/v kernel.
-// step_path 1 runs one kernel per op with rocBLAS linear layers; all round to fp16 at the
-// same points.  With `graph` the
+// (kvc_block_qkv / swiglu / linear), with the prompts' K/V stored by the q/k/v kernel, and
+// rocBLAS with one kernel per op for the products where that is faster (fused_products).
+// step_path 1 runs every op as a kernel of its own; all round to fp16 at the same points.  With `graph` the
 // fused step is captured once as a HIP graph whose kernels read the step's counts
 // (rows, attention units, partial records) from device memory; each step then
 // uploads its metadata into fixed places and replays the graph (the reference
@@ -208,47 +208,72 @@ struct QwenModel {
     void* kl(int l) const { return kvm.k_layer(l); }
     void* vl(int l) const { return kvm.v_layer(l); }
 
+    // Which products of a many-row layer run as one fused kernel (kvc_block_*) and which as
+    // rocBLAS and a kernel per op (us, op by op and fused).  Large products of wide layers
+    // belong to rocBLAS: gate|up at 1024 rows of hidden 2048 110 and 149, at 128 of 4096 72 and
+    // 56; o_proj at 1500 rows of 1536 17 and 20, at 4096 of 896 16.9 and 16.1 (few rows are level
+    // alone, but in a layer each launch saved counts: 256 rows of 4096 282 and 262 in all); q|k|v,
+    // with five more launches, later: 2048 rows of 4096 149 and 133, 3000 185 and 213.  down_proj
+    // follows its rows: up to about 1400 the fused kernel's K groups fill the chip (inter 4864,
+    // 700 rows 28.5 and 20.5; 11008, 1024 rows 111 and 86; 4864, 3000 rows 38 and 67), and a K
+    // of some 5000 is the longer chain at few rows (64 rows 11.8 and 18.6, 384 rows 33 and 20).
+    struct Fused { bool qkv, o, gate_up, down; };
+    Fused fused_products(int M) const {
+        const double H = c.hidden, QD = (double)c.n_heads * c.head_dim, KD = (double)c.n_kv_heads * c.head_dim;
+        const double I = c.inter;
+        Fused f{};
+        if (!block_ok) return f;
+        f.qkv = M * (QD + 2 * KD) * H <= 45e9;
+        f.o = QD <= 1024 || M <= 320 || (QD <= 2048 && M * H * QD <= 2.4e9);
+        f.gate_up = H <= 1024 || M <= 320 || M * 2 * I * H <= 16e9;
+        f.down = M <= 1400 && (I >= 6144 || (I >= 3072 && M >= 320));
+        return f;
+    }
+
     // Rows [0, M) of x hold the layer input; attention is supplied by attend(l, written),
-    // `written` when the rows' K/V already lie in the pools (fused path with d_slots).
+    // `written` when the rows' K/V already lie in the pools (fused q|k|v with d_slots).
     template <typename Attend>
     void layers(int M, const int* d_pos, int pos_base, const int* d_slots, Attend&& attend) {
         const int H = c.hidden, QD = c.n_heads * c.head_dim, KD = c.n_kv_heads * c.head_dim, I = c.inter;
-        if (block_ok) {
-            for (int l = 0; l < c.layers; ++l) {
-                const Layer& w = L[l];
-                kvc::check(kvc_rmsnorm(nrm, x, w.ln1, M, H, c.eps, stream), "rmsnorm");
+        const Fused f = fused_products(M);
+        for (int l = 0; l < c.layers; ++l) {
+            const Layer& w = L[l];
+            kvc::check(kvc_rmsnorm(nrm, x, w.ln1, M, H, c.eps, stream), "rmsnorm");
+            if (f.qkv) {
                 kvc::check(kvc_block_qkv(q, d_slots ? kl(l) : k, d_slots ? vl(l) : v, nrm, w.wq, w.bq, d_pos, pos_base,
                                          d_slots, M, H, c.n_heads, c.n_kv_heads, c.head_dim, c.block_size, c.theta,
                                          stream),
                            "qkv + bias + rope");
-                attend(l, d_slots != nullptr);
-                kvc::check(kvc_block_linear(x, att, w.wo, M, H, QD, 1, stream), "o_proj + residual");
-                kvc::check(kvc_rmsnorm(nrm, x, w.ln2, M, H, c.eps, stream), "rmsnorm");
-                kvc::check(kvc_block_swiglu(gate, nrm, w.wg, M, I, H, stream), "gate/up + swiglu");
-                kvc::check(kvc_block_linear(x, gate, w.wd, M, H, I, 1, stream), "down_proj + residual");
+            } else {
+                kvc::check(kvc_linear(q, nrm, w.wq, M, QD, H, KVC_F16, stream), "q_proj");
+                kvc::check(kvc_add_bias(q, w.bq, M, QD, stream), "q bias");
+                kvc::check(kvc_linear(k, nrm, w.wk, M, KD, H, KVC_F16, stream), "k_proj");
+                kvc::check(kvc_add_bias(k, w.bk, M, KD, stream), "k bias");
+                kvc::check(kvc_linear(v, nrm, w.wv, M, KD, H, KVC_F16, stream), "v_proj");
+                kvc::check(kvc_add_bias(v, w.bv, M, KD, stream), "v bias");
+                kvc::check(kvc_rope(q, d_pos, pos_base, M, c.n_heads, c.head_dim, c.theta, stream), "rope q");
+                kvc::check(kvc_rope(k, d_pos, pos_base, M, c.n_kv_heads, c.head_dim, c.theta, stream), "rope k");
             }
-            return;
-        }
-        for (int l = 0; l < c.layers; ++l) {
-            const Layer& w = L[l];
-            kvc::check(kvc_rmsnorm(nrm, x, w.ln1, M, H, c.eps, stream), "rmsnorm");
-            kvc::check(kvc_linear(q, nrm, w.wq, M, QD, H, KVC_F16, stream), "q_proj");
-            kvc::check(kvc_add_bias(q, w.bq, M, QD, stream), "q bias");
-            kvc::check(kvc_linear(k, nrm, w.wk, M, KD, H, KVC_F16, stream), "k_proj");
-            kvc::check(kvc_add_bias(k, w.bk, M, KD, stream), "k bias");
-            kvc::check(kvc_linear(v, nrm, w.wv, M, KD, H, KVC_F16, stream), "v_proj");
-            kvc::check(kvc_add_bias(v, w.bv, M, KD, stream), "v bias");
-            kvc::check(kvc_rope(q, d_pos, pos_base, M, c.n_heads, c.head_dim, c.theta, stream), "rope q");
-            kvc::check(kvc_rope(k, d_pos, pos_base, M, c.n_kv_heads, c.head_dim, c.theta, stream), "rope k");
-            attend(l, false);
-            kvc::check(kvc_linear(o, att, w.wo, M, H, QD, KVC_F16, stream), "o_proj");
-            kvc::check(kvc_add_residual(x, o, (size_t)M * H, stream), "residual");
+            attend(l, f.qkv && d_slots != nullptr);
+            project_residual(f.o, att, w.wo, M, QD, "o_proj + residual");
             kvc::check(kvc_rmsnorm(nrm, x, w.ln2, M, H, c.eps, stream), "rmsnorm");
-            kvc::check(kvc_linear(gate, nrm, w.wg, M, I, H, KVC_F16, stream), "gate_proj");
-            kvc::check(kvc_linear(up, nrm, w.wu, M, I, H, KVC_F16, stream), "up_proj");
-            kvc::check(kvc_silu_mul(gate, gate, up, (size_t)M * I, stream), "silu");
-            kvc::check(kvc_linear(o, gate, w.wd, M, H, I, KVC_F16, stream), "down_proj");
-            kvc::check(kvc_add_residual(x, o, (size_t)M * H, stream), "residual");
+            if (f.gate_up) {
+                kvc::check(kvc_block_swiglu(gate, nrm, w.wg, M, I, H, stream), "gate/up + swiglu");
+            } else {
+                kvc::check(kvc_linear(gate, nrm, w.wg, M, I, H, KVC_F16, stream), "gate_proj");
+                kvc::check(kvc_linear(up, nrm, w.wu, M, I, H, KVC_F16, stream), "up_proj");
+                kvc::check(kvc_silu_mul(gate, gate, up, (size_t)M * I, stream), "silu");
+            }
+            project_residual(f.down, gate, w.wd, M, I, "down_proj + residual");
+        }
+    }
+    // x += a W^T over M rows
+    void project_residual(bool fused, const void* a, const void* w, int M, int K, const char* what) {
+        if (fused) {
+            kvc::check(kvc_block_linear(x, a, w, M, c.hidden, K, 1, stream), what);
+        } else {
+            kvc::check(kvc_linear(o, a, w, M, c.hidden, K, KVC_F16, stream), what);
+            kvc::check(kvc_add_residual(x, o, (size_t)M * c.hidden, stream), what);
         }
     }
 
