@@ -329,9 +329,10 @@ int kvc_batched_paged_decode_planned_dev(const void* q, const void* k_new, const
 /* qk_paged_causal_attn (qwen_kernels.h:19-21, qwen_kernels.cu:146-181): the prompt
  * (prefill) attention of one sequence.  Query i of q [Nq, Hq, D] sits at position
  * q_pos_base + i and attends causally to positions 0 .. q_pos_base + i of the
- * paged pools through block_table; out is [Nq, Hq, D].  Runs the batched decode
- * kernels with query i as a sequence of length q_pos_base + i + 1 sharing the one
- * table (grouped-query heads on the matrix cores, long prefixes split and merged).
+ * paged pools through block_table; out is [Nq, Hq, D].  fp16, head_dim 64 or 128 and a
+ * power-of-two BLOCK >= 16 run the tiled matrix-core kernels (32 to 128 queries per key
+ * tile, few queries behind long prefixes split and merged); other shapes the batched decode
+ * kernels with query i as a sequence of length q_pos_base + i + 1 sharing the one table.
  * workspace as for the batched decode (NULL: library-owned). */
 int kvc_paged_causal_attn(const void* q, void* out, const void* k_pool, const void* v_pool, const int* block_table,
                           int q_pos_base, int Nq, int Hq, int Hkv, int D, int BLOCK, float scale, int dtype,

@@ -1071,9 +1071,10 @@ int launch_gqa_mode(DecodeLaunch L, dim3 grid, hipStream_t st) {
         case kPagedUniform:   L.lds_pad = lds_pad(gqa_mfma_kernel<D, kPagedUniform, WPB>, L.wg_per_cu); hipLaunchKernelGGL((gqa_mfma_kernel<D, kPagedUniform, WPB>), grid, block, L.lds_pad, st, L.p.work, L.p.work_ints, L.p); break;
         case kPlannedUniform: L.lds_pad = lds_pad(gqa_mfma_kernel<D, kPlannedUniform, WPB>, L.wg_per_cu); hipLaunchKernelGGL((gqa_mfma_kernel<D, kPlannedUniform, WPB>), grid, block, L.lds_pad, st, L.p.work, L.p.work_ints, L.p); break;
         case kCausalTile:
-            if (L.qtile == 128) hipLaunchKernelGGL((prompt_kernel<D, 4, 8>), grid, dim3(8 * kWave), 0, st, L.p);
-            else if (L.qtile == 64) hipLaunchKernelGGL((prompt_kernel<D, 2, 8>), grid, dim3(8 * kWave), 0, st, L.p);
-            else hipLaunchKernelGGL((prompt_stream_kernel<D, 1>), grid, dim3(8 * kWave), 0, st, L.p);
+            if (L.qtile == 32) hipLaunchKernelGGL((prompt_stream_kernel<D>), grid, dim3(8 * kWave), 0, st, L.p);
+            else if (L.qtile == 64) hipLaunchKernelGGL((prompt_kernel<D, 2>), grid, dim3(8 * kWave), 0, st, L.p);
+            else if constexpr (D == 128) hipLaunchKernelGGL((prompt_kernel<D, 4>), grid, dim3(8 * kWave), 0, st, L.p);
+            else return set_error(KVC_ERR_UNSUPPORTED, "prompt attention: tiles of 128 queries need head_dim 128");
             break;
         case kSelfPlanned:
             L.lds_pad = lds_pad(gqa_mfma_kernel<D, kSelfPlanned, WPB>, L.wg_per_cu);

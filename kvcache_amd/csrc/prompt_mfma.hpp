@@ -91,8 +91,9 @@ __device__ __forceinline__ f32x4 add_nonfinite(f32x4 acc, const char* vb, const 
     return acc;
 }
 
-template <int D, int QG, int W>
-__global__ __launch_bounds__(W * kWave) void prompt_kernel(DecodeParams p) {
+template <int D, int QG>
+__global__ __launch_bounds__(8 * kWave) void prompt_kernel(DecodeParams p) {
+    constexpr int W = 8;
     constexpr int ROW = D * 2;              // bytes per K/V row
     constexpr int KS = W / QG;              // key streams
     constexpr int kPromptSet = 16 * W;      // keys per LDS set (each wave loads 16 rows)
@@ -347,11 +348,11 @@ __global__ __launch_bounds__(W * kWave) void prompt_kernel(DecodeParams p) {
     }
 }
 
-// Key streams of their own: wave w of 8 takes key tiles w, w + 8, ... of 32
-// keys for all 32 * NC queries of the workgroup, loading and staging them by itself, so no
-// barrier holds the waves in step (where every wave meets the same unit at once: loads,
-// then LDS writes, then MFMAs) and a K/V fragment read from LDS serves NC column tiles.
-template <int D, int NC>
+// Key streams of their own: wave w of 8 takes key tiles w, w + 8, ... of 32 keys for the 32
+// queries of the workgroup, loading and staging them by itself, so no barrier holds the
+// waves in step (where every wave meets the same unit at once: loads, then LDS writes, then
+// MFMAs).
+template <int D>
 __global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kernel(DecodeParams p) {
     constexpr int ROW = D * 2;
     constexpr int KD = D / 16, DT = D / 32;
@@ -359,7 +360,7 @@ __global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kern
     constexpr int W = 8;
     constexpr int kTile = 32 * ROW;          // bytes of one K (or V) tile
     __shared__ __attribute__((aligned(16))) char s_kv[W][2][kTile];
-    __shared__ float s_ml[W][32 * NC][2];
+    __shared__ float s_ml[W][32][2];
 
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = uniform(threadIdx.x >> 6);
@@ -367,8 +368,8 @@ __global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kern
     int unit = blockIdx.x;
     const int hi = unit % p.Hq;  unit /= p.Hq;
     const int hk = hi % p.Hkv, qh = hk * p.group + hi / p.Hkv;
-    const int ntq = (p.N + 32 * NC - 1) / (32 * NC);
-    const int q0 = (ntq - 1 - unit % ntq) * 32 * NC;
+    const int ntq = (p.N + 31) / 32;
+    const int q0 = (ntq - 1 - unit % ntq) * 32;
     const int c = unit / ntq;
     // the position and, with it, the chunks: from the host, or from device memory
     int base = p.fixed_len, chunk = p.chunk_tokens;
@@ -380,7 +381,7 @@ __global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kern
         const long long M63 = (long long)(p.sp_records - 1) * p.sp_max_chunk;
         if (2LL * base + p.N + 1 > 2 * M63 || (p.sp_nc_max && lall > 63LL * p.sp_max_chunk)) {
             if (c == 0) {
-                for (int q = q0; q < min(q0 + 32 * NC, p.N); ++q) {
+                for (int q = q0; q < min(q0 + 32, p.N); ++q) {
                     _Float16* ob = static_cast<_Float16*>(p.out) + ((size_t)q * p.Hq + qh) * D;
                     for (int e = threadIdx.x; e < D; e += W * kWave) ob[e] = (_Float16)__builtin_nanf("");
                 }
@@ -392,7 +393,7 @@ __global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kern
         const int al = max(p.block, 256);
         chunk = max((lall / nch + al) / al * al, al);  // nch chunks of it cover lall
     }
-    const int lmax = base + min(q0 + 32 * NC, p.N);
+    const int lmax = base + min(q0 + 32, p.N);
     const int j0 = c * chunk, j1 = min(j0 + chunk, lmax);
     if (j0 >= lmax && c > 0) return;
     const int ntiles = max(0, j1 - j0 + 31) / 32;  // (none: a position below -q, whose rows are 0)
@@ -441,34 +442,24 @@ __global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kern
 
     load_ids(0);
     issue(0);
-    f16x8v qb[NC][KD];
+    f16x8v qb[KD];
     {
         const __amdgpu_buffer_rsrc_t qr = tile_rsrc(p.q, p.N * p.Hq * ROW);
+        const int qoff = ((q0 + l32) * p.Hq + qh) * ROW + h * 16;
 #pragma unroll
-        for (int n = 0; n < NC; ++n) {
-            const int qoff = ((q0 + 32 * n + l32) * p.Hq + qh) * ROW + h * 16;
-#pragma unroll
-            for (int d = 0; d < KD; ++d) qb[n][d] = __builtin_bit_cast(f16x8v, buffer_load16(qr, qoff + d * 32));
-        }
+        for (int d = 0; d < KD; ++d) qb[d] = __builtin_bit_cast(f16x8v, buffer_load16(qr, qoff + d * 32));
     }
     const float sl2 = fabsf(p.scale_log2);
     if (p.scale_log2 < 0.f) {
 #pragma unroll
-        for (int n = 0; n < NC; ++n)
-#pragma unroll
-            for (int d = 0; d < KD; ++d) qb[n][d] = -qb[n][d];
+        for (int d = 0; d < KD; ++d) qb[d] = -qb[d];
     }
-    float m[NC], l[NC], top[NC];  // as prompt_kernel's
-    f32x16 O[NC][DT];
+    float m = -FLT_MAX, l = 0.f, top = -FLT_MAX;  // as prompt_kernel's
+    f32x16 O[DT];
 #pragma unroll
-    for (int n = 0; n < NC; ++n) {
-        m[n] = top[n] = -FLT_MAX;
-        l[n] = 0.f;
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) O[n][dt][i] = 0.f;
-    }
+        for (int i = 0; i < 16; ++i) O[dt][i] = 0.f;
     int ka[4], va[DT];
 #pragma unroll
     for (int d = 0; d < 4; ++d) ka[d] = l32 * ROW + kchunk(l32, 2 * d + h) * 16;
@@ -478,55 +469,48 @@ __global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kern
 
     auto compute = [&](int t0, auto masked_tag) {
         constexpr bool MASKED = decltype(masked_tag)::value;
-        f32x16 S[NC];
+        f32x16 S;
 #pragma unroll
-        for (int n = 0; n < NC; ++n)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) S[n][i] = 0.f;
+        for (int i = 0; i < 16; ++i) S[i] = 0.f;
 #pragma unroll
         for (int d = 0; d < KD; ++d) {
             const f16x8v a = *reinterpret_cast<const f16x8v*>(kt + ka[d & 3] + (d >> 2) * 128);
-#pragma unroll
-            for (int n = 0; n < NC; ++n) S[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qb[n][d], S[n], 0, 0, 0);
+            S = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, qb[d], S, 0, 0, 0);
         }
-        f16x8v pb[NC][2];
+        f16x8v pb[2];
+        const int lim = base + q0 + l32 - t0 - 4 * h;
+        auto seen = [&](int i) { return !MASKED || 8 * (i >> 2) + (i & 3) <= lim; };
+        float mx = -FLT_MAX;
 #pragma unroll
-        for (int n = 0; n < NC; ++n) {
-            const int lim = base + q0 + 32 * n + l32 - t0 - 4 * h;
-            auto seen = [&](int i) { return !MASKED || 8 * (i >> 2) + (i & 3) <= lim; };
-            float mx = -FLT_MAX;
+        for (int i = 0; i < 16; ++i) mx = seen(i) ? fmaxf(mx, S[i]) : mx;
+        mx = max_xor32(mx) * sl2;
+        if (__any(mx > (D == 128 ? top : m))) {
+            if constexpr (D == 128) top = fmaxf(top, mx);
+            const float mn = D == 128 ? fmaxf(mx, top - 8.f) : fmaxf(m, mx);
+            const float corr = fast_exp2(m - mn);
+            m = mn;
+            l *= corr;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) mx = seen(i) ? fmaxf(mx, S[n][i]) : mx;
-            mx = max_xor32(mx) * sl2;
-            if (__any(mx > (D == 128 ? top[n] : m[n]))) {
-                if constexpr (D == 128) top[n] = fmaxf(top[n], mx);
-                const float mn = D == 128 ? fmaxf(mx, top[n] - 8.f) : fmaxf(m[n], mx);
-                const float corr = fast_exp2(m[n] - mn);
-                m[n] = mn;
-                l[n] *= corr;
+            for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-                for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) O[n][dt][i] *= corr;
-            }
-            float ps = 0.f;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                float e = fast_exp2(__builtin_fmaf(S[n][i], sl2, -m[n]));
-                e = seen(i) ? e : 0.f;
-                ps += e;
-                pb[n][i >> 3][i & 7] = (_Float16)e;
-            }
-            l[n] += ps;
+                for (int i = 0; i < 16; ++i) O[dt][i] *= corr;
         }
+        float ps = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            float e = fast_exp2(__builtin_fmaf(S[i], sl2, -m));
+            e = seen(i) ? e : 0.f;
+            ps += e;
+            pb[i >> 3][i & 7] = (_Float16)e;
+        }
+        l += ps;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) {
                 const s16x4v lo = ds_read_tr16(vt + va[dt] + 16 * t * ROW), hi2 = ds_read_tr16(vt + va[dt] + (16 * t + 8) * ROW);
                 const f16x8v a = __builtin_bit_cast(f16x8v, __builtin_shufflevector(lo, hi2, 0, 1, 2, 3, 4, 5, 6, 7));
-#pragma unroll
-                for (int n = 0; n < NC; ++n) O[n][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb[n][t], O[n][dt], 0, 0, 0);
+                O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb[t], O[dt], 0, 0, 0);
             }
     };
     bool bad = false;  // this wave cleared elements of V in its tiles of the causal edge
@@ -558,29 +542,24 @@ __global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kern
 
     // combine: every wave's O through LDS, then wave w sums its share of the slots of four
     // consecutive dims of a column (a slot: 64 lanes x 4 dims)
-    constexpr int kSlots = NC * DT * 4;
+    constexpr int kSlots = DT * 4;
     constexpr int kPer = kSlots / W;
     static_assert(kSlots % W == 0 && W * kSlots * kWave * 16 <= (int)sizeof(s_kv), "the partials fit the tiles");
     f32x4* part = reinterpret_cast<f32x4*>(&s_kv[0][0][0]);
     __syncthreads();
     const int nw = min(W, ntiles);  // waves that had tiles
     if (wave < max(nw, 2) || nw > 2) {
-#pragma unroll
-        for (int n = 0; n < NC; ++n) {
-            const float lt = sum_xor32(l[n]);
-            if (h == 0) {
-                s_ml[wave][32 * n + l32][0] = m[n];
-                s_ml[wave][32 * n + l32][1] = bad ? -lt : lt;  // (the sign, also of 0: elements to add)
-            }
-#pragma unroll
-            for (int i = 0; i < DT * 4; ++i)
-                part[((wave * NC + n) * DT * 4 + i) * kWave + lane] =
-                    f32x4{O[n][i >> 2][4 * (i & 3)], O[n][i >> 2][4 * (i & 3) + 1], O[n][i >> 2][4 * (i & 3) + 2],
-                          O[n][i >> 2][4 * (i & 3) + 3]};
+        const float lt = sum_xor32(l);
+        if (h == 0) {
+            s_ml[wave][l32][0] = m;
+            s_ml[wave][l32][1] = bad ? -lt : lt;  // (the sign, also of 0: elements to add)
         }
+#pragma unroll
+        for (int i = 0; i < kSlots; ++i)
+            part[(wave * kSlots + i) * kWave + lane] =
+                f32x4{O[i >> 2][4 * (i & 3)], O[i >> 2][4 * (i & 3) + 1], O[i >> 2][4 * (i & 3) + 2], O[i >> 2][4 * (i & 3) + 3]};
     }
     __syncthreads();
-    const int n = NC == 1 ? 0 : wave * kPer / (DT * 4), col = 32 * n + l32;
     float M = -FLT_MAX, lt = 0.f;
     unsigned any_bad = 0;
     f32x4 acc[kPer];
@@ -591,12 +570,12 @@ __global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kern
         float mw[NW];
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            mw[w] = s_ml[w][col][0];
+            mw[w] = s_ml[w][l32][0];
             M = fmaxf(M, mw[w]);
         }
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            const float wk = fast_exp2(mw[w] - M), lw = s_ml[w][col][1];
+            const float wk = fast_exp2(mw[w] - M), lw = s_ml[w][l32][1];
             any_bad |= __float_as_uint(lw) & 0x80000000u;
             lt = __builtin_fmaf(wk, fabsf(lw), lt);
 #pragma unroll
@@ -610,13 +589,13 @@ __global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kern
     // prompts of up to 64 keys leave two waves' partials (8 queries: 5.0 us with all eight, 4.5)
     if (nw > 2) combine(std::integral_constant<int, W>{});
     else combine(std::integral_constant<int, 2>{});
-    const int q = q0 + col;
+    const int q = q0 + l32;
     const int ncq = max(base + q, 0) / chunk + 1;  // chunks of the query
     if (any_bad)
 #pragma unroll
         for (int i = 0; i < kPer; ++i)
             acc[i] = add_nonfinite<D>(acc[i], vb, p.table_all, bsh, p.Hkv, hk, j0 + 32 * full, min(base + q, j1 - 1),
-                                      8 * ((wave * kPer + i) % (DT * 4)) + 4 * h);
+                                      8 * (wave * kPer + i) + 4 * h);
     // host positions: merge_kernel follows (20 queries, 14 heads, behind 5900 keys: 10.5 us,
     // 13.9 merged in here); a device position does not know on the host whether one is needed
     const bool fused = p.merge_mode == kMergeAtomic;
@@ -625,7 +604,7 @@ __global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kern
         const size_t rec = ((size_t)q * p.max_chunks + c) * p.Hq + qh;
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
-            const int d0 = 8 * ((wave * kPer + i) % (DT * 4)) + 4 * h;
+            const int d0 = 8 * (wave * kPer + i) + 4 * h;
             if (ncq == 1) {
                 f16x4 o;
 #pragma unroll
@@ -652,12 +631,12 @@ __global__ __launch_bounds__(8 * kWave, D == 64 ? 4 : 2) void prompt_stream_kern
     __builtin_amdgcn_s_waitcnt(0);  // every thread's partial stores complete before the arrival
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __syncthreads();
-    unsigned long long* ctr = p.counters + ctr_slot((size_t)(q0 / (32 * NC)) * p.Hq + qh, p.ctr_shift);
+    unsigned long long* ctr = p.counters + ctr_slot((size_t)(q0 / 32) * p.Hq + qh, p.ctr_shift);
     if (threadIdx.x == 0) s_last = arrive(ctr, p.epoch) == (unsigned)(nct - 1);
     __syncthreads();
     if (!s_last) return;
     auto ld = [](const float* a) { return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
-    for (int i = threadIdx.x; i < 32 * NC * (D / 4); i += W * kWave) {
+    for (int i = threadIdx.x; i < 32 * (D / 4); i += W * kWave) {
         const int qm = q0 + i / (D / 4), d0 = i % (D / 4) * 4;
         const int nm = max(base + qm, 0) / chunk + 1;
         if (qm >= p.N || nm == 1) continue;

@@ -502,6 +502,7 @@ __global__ __launch_bounds__(WAVES * 64) void rows_kernel(RowsParams p) {
     const int M = uniform(p.dev_rows ? min(max(*p.dev_rows, 0), p.M) : p.M);
     constexpr int kThreads = WAVES * 64;
     constexpr int kItems = kRows * 16 / kThreads;  // (row, column pair) items per thread
+    static_assert(EPI != kEpiLogits || !SPLIT, "a candidate needs whole rows (a split group's early workgroups have none)");
     __shared__ float s_red[2][WAVES][kRows][kCols + 1];
     __shared__ float s_ss[WAVES][kRows];
     __shared__ unsigned s_last;
@@ -979,8 +980,11 @@ Shape plan_shape(int groups, int K, bool norm) {
     int shape = g_tune_shape;
     // automatic: 8x4 while one workgroup covers K (gate|up at I 4864, 304 groups: 7.1 us
     // vs 7.8 us at 4x7; lm_head at 32 rows, 1536 / 3136 / 4748 / 8192 groups: 21.3 / 45.2
-    // / 64.2 / 110.2 us vs 22.3 / 47.5 / 66.8 / 114.4 us), 8x4 with K split past 32 steps
-    // (down_proj K 4864 at 32 rows: 5 splits)
+    // / 64.2 / 110.2 us vs 22.3 / 47.5 / 66.8 / 114.4 us; at one row, 1000 / 1536 / 3136 / 4748
+    // groups: 14.9 / 18.9 / 31.7 / 45.4 us vs 16.8 / 25.8 / 41.9 / 56.4 us at 4x7 and two
+    // workgroups per CU; gate|up of I 16640, 1040 groups, 13.6 vs 15.7 us, behind only at K 512
+    // from 2048 groups on, 15.8 vs 14.6 us), 8x4 with K split past 32 steps (down_proj K 4864
+    // at 32 rows: 5 splits)
     if (shape < 0) shape = ks <= 32 ? 1 : 3;
     if (shape == 0 && ks > 28) shape = 1;
     if (shape == 1 && ks > 32) shape = 2;
@@ -1020,10 +1024,12 @@ int launch_rows(RowsParams p, const Shape& s, hipStream_t st) {
         if (two) hipLaunchKernelGGL((rows_kernel<EPI, NORM, 2, W, S, SPLIT>), grid, dim3(W * 64), 0, st, p);   \
         else hipLaunchKernelGGL((rows_kernel<EPI, NORM, 1, W, S, SPLIT>), grid, dim3(W * 64), 0, st, p);       \
     } while (0)
-    if (s.waves == 8 && s.splits > 1) KVC_ROWS_LAUNCH(8, 4, true);
-    else if (s.waves == 8) KVC_ROWS_LAUNCH(8, 4, false);
+    if (s.splits > 1) {
+        if constexpr (EPI == kEpiLogits) return set_error(KVC_ERR_UNSUPPORTED, "rows lm_head: no K split");
+        else if (s.waves == 8) KVC_ROWS_LAUNCH(8, 4, true);
+        else KVC_ROWS_LAUNCH(4, 4, true);
+    } else if (s.waves == 8) KVC_ROWS_LAUNCH(8, 4, false);
     else if (s.steps == 7) KVC_ROWS_LAUNCH(4, 7, false);
-    else if (s.splits > 1) KVC_ROWS_LAUNCH(4, 4, true);
     else KVC_ROWS_LAUNCH(4, 4, false);
 #undef KVC_ROWS_LAUNCH
     return hip_check(hipGetLastError(), "rows linear launch");
