@@ -516,3 +516,29 @@ def test_block_swiglu(M_, I, H):
     ops.block_swiglu(act, dev(x), dev(w), M_, I, H)
     g, u = _r16(M.linear(x.astype(np.float32), w[:I])), _r16(M.linear(x.astype(np.float32), w[I:]))
     close(host(act, np.float16, (M_, I)), M.silu_mul(g, u))
+
+
+def test_block_refuses_bad_calls():
+    say("block linear layers: argument errors")
+    from kvcache_amd import KvcError
+    x, w, y, b = (DeviceBuffer(1 << 20) for _ in range(4))
+    refused = [
+        lambda: ops.block_linear(y, x, w, 4, 12, 64),             # N not a multiple of 8
+        lambda: ops.block_linear(y, x, w, 4, 16, 12),             # K not a multiple of 8
+        lambda: ops.block_linear(y, x, w, -1, 16, 16),
+        lambda: ops.block_linear(x, x, w, 4, 16, 16),             # y is x
+        lambda: ops.block_linear(y.ptr + 8, x, w, 4, 16, 16),     # misaligned
+        lambda: ops.block_linear(y, x.ptr + 2, w, 4, 16, 16),
+        lambda: ops.block_linear(y, None, w, 4, 16, 16),
+        lambda: ops.block_swiglu(y, x, w, 4, 12, 64),
+        lambda: ops.block_swiglu(y.ptr + 4, x, w, 4, 16, 64),
+        lambda: ops.block_qkv(y, y, y, x, w, b, 4, 64, 2, 1, 48, 1e6),              # head_dim
+        lambda: ops.block_qkv(y, y, y, x, w, b, 4, 64, 2, 1, 64, 1.0),              # theta
+        lambda: ops.block_qkv(y, y, y, x, w, b, 4, 60, 2, 1, 64, 1e6),              # hidden
+        lambda: ops.block_qkv(y, y, y, x, w, None, 4, 64, 2, 1, 64, 1e6),           # no bias
+        lambda: ops.block_qkv(y, y, y, x, w, b, 4, 64, 2, 1, 64, 1e6, slots=b),     # slots without BLOCK
+    ]
+    for call in refused:
+        with pytest.raises(KvcError):
+            call()
+    ops.block_linear(y, x, w, 0, 16, 16)  # no rows: nothing to do

@@ -450,3 +450,100 @@ def test_short_grouped_batches_stay_whole(orc, D, Hq, Hkv, longest):
     np.testing.assert_array_equal(got, host(out, np.float16, q.shape))
     ref = orc.batched_paged(q, kp, vp, table, off, lens, Hkv, B, scale)
     assert np.abs(got.astype(np.float64) - ref).max() <= tol(KVC_F16)
+
+
+# ---- prompt queries at a device position in prompt_stream_kernel (8 grouped queries and more) ----
+def prompt_chunk(base, n, Hq, D):
+    """The kernel's chunk of keys (prompt_stream_kernel, blocks of 16 tokens)."""
+    lall = base + n
+    nch = 1 if lall < 3072 else min(max(lall // (512 if D == 64 else 1024), 1), min(64, max(1, 256 // ((n + 31) // 32 * Hq))))
+    return (lall // nch + 256) // 256 * 256
+
+
+def split_bases(n, Hq, D):
+    """Positions: whole; a chunk's edge between the first and the last query; few and many chunks."""
+    edges = [b for b in range(3200, 9000) if (b + n // 2) % prompt_chunk(b, n, Hq, D) == 0]
+    return [700, 3072 - n, edges[0], edges[-1] + 1, 5 * 1024]
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,n", [(64, 14, 2, 8), (64, 14, 2, 70), (128, 8, 2, 8), (128, 8, 2, 40), (128, 16, 1, 33)])
+def test_device_position_merges_in_the_launch(orc, D, Hq, Hkv, n):
+    # split prefixes: partials, arrival counter, last arriver's merge and its counter's reset, call
+    # after call on one workspace, without one where the static scratch allows, and as one captured
+    # launch replayed at every position with eager calls on the same workspace between
+    import ctypes as C
+
+    from kvcache_amd._native import check, lib
+    say(f"device position, merge in the launch D={D} Hq={Hq} Hkv={Hkv} n={n}")
+    B, L = 16, lib()
+    bases = split_bases(n, Hq, D)
+    assert any(b // prompt_chunk(b, n, Hq, D) != (b + n - 1) // prompt_chunk(b, n, Hq, D) for b in bases)
+    nb = (max(bases) + n + B - 1) // B
+    table = np.random.default_rng(n).permutation(nb).astype(np.int32)
+    kp, vp = normal((nb, Hkv, B, D), 300, np.float16), normal((nb, Hkv, B, D), 301, np.float16)
+    q = normal((n, Hq, D), 302, np.float16)
+    scale = float(1.0 / np.sqrt(D))
+    dq, dk, dv, dt = dev(q), dev(kp), dev(vp), dev(table)
+    pos, out = dev(np.array([0], np.int32)), DeviceBuffer(q.nbytes)
+    ws = DeviceBuffer(int(L.kvc_paged_causal_attn_dev_workspace_size(n, Hq, Hkv, D, B, KVC_F16)))
+    want = {b: orc.batched_paged(q, kp, vp, table, np.zeros(n + 1, np.int32), b + 1 + np.arange(n, dtype=np.int32), Hkv, B,
+                                 scale, nthreads=8) for b in bases}
+
+    def call(stream=None, noalloc=False):
+        if noalloc:
+            check(L.kvc_paged_causal_attn_dev_noalloc(dq.ptr, out.ptr, dk.ptr, dv.ptr, dt.ptr, pos.ptr, n, Hq, Hkv, D, B,
+                                                      C.c_float(scale), KVC_F16, stream))
+        else:
+            check(L.kvc_paged_causal_attn_dev(dq.ptr, out.ptr, dk.ptr, dv.ptr, dt.ptr, pos.ptr, n, Hq, Hkv, D, B,
+                                              C.c_float(scale), KVC_F16, ws.ptr, ws.nbytes, stream))
+
+    def result():
+        return host(out, np.float16, q.shape)
+
+    eager = {}
+    for b in bases + bases[::-1]:
+        pos.upload(np.array([b], np.int32))
+        call()
+        got = result()
+        assert np.abs(got.astype(np.float64) - want[b]).max() <= tol(KVC_F16), b
+        np.testing.assert_array_equal(got, eager.setdefault(b, got))
+        if n == 8:
+            call(noalloc=True)
+            np.testing.assert_array_equal(result(), got)
+    st, ex = C.c_void_p(), C.c_void_p()
+    check(L.kvc_stream_create(C.byref(st)))
+    check(L.kvc_graph_begin(st))
+    call(st)
+    check(L.kvc_graph_end(st, C.byref(ex)))
+    for b in bases * 2:
+        pos.upload(np.array([b], np.int32))
+        check(L.kvc_graph_launch(ex, st))
+        check(L.kvc_stream_synchronize(st))
+        np.testing.assert_array_equal(result(), eager[b])
+        call()  # (the same counters under another call's epoch)
+        np.testing.assert_array_equal(result(), eager[b])
+    check(L.kvc_graph_destroy(ex))
+    check(L.kvc_stream_destroy(st))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_device_position_outside_the_keys(orc, D):
+    # queries at negative positions have no keys (zero rows); a position past the planning budget
+    # gives NaN rows and a report, and reads nothing
+    say(f"device position negative and past the budget D={D}")
+    Hq, Hkv, B, n = 8, 2, 16, 9
+    kp, vp = normal((2, Hkv, B, D), 310, np.float16), normal((2, Hkv, B, D), 311, np.float16)
+    q = normal((n, Hq, D), 312, np.float16)
+    table, pos, out = np.array([1, 0], np.int32), dev(np.array([0], np.int32)), DeviceBuffer(q.nbytes)
+    for base in (-4, -40):
+        pos.upload(np.array([base], np.int32))
+        ops.qkcuda_paged_causal_attn(dev(q), out, dev(kp), dev(vp), dev(table), pos, n, Hq, Hkv, D, B, 0.125)
+        got = host(out, np.float16, q.shape)
+        lens = np.maximum(base + 1 + np.arange(n), 0).astype(np.int32)
+        want = orc.batched_paged(q, kp, vp, table, np.zeros(n + 1, np.int32), lens, Hkv, B, 0.125)
+        assert np.all(got[lens == 0] == 0)
+        assert np.abs(got.astype(np.float64) - want)[lens > 0].max(initial=0) <= tol(KVC_F16)
+    pos.upload(np.array([63 * 1024 * B], np.int32))
+    ops.qkcuda_paged_causal_attn(dev(q), out, dev(kp), dev(vp), dev(table), pos, n, Hq, Hkv, D, B, 0.125)
+    assert np.isnan(host(out, np.float16, q.shape)).all()
+    expect_device_error()
