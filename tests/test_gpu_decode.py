@@ -496,8 +496,8 @@ def test_paged_causal_attn(orc, dtype, Hq, Hkv, base, n):
 
 
 # the tiles of the prompt kernels: 32 queries (few workgroups), 64 (D 64 from 512 workgroups
-# of them, D 128 from 160), 128 (D 128 from 160); keys in sets of 128 or streams of 256, the
-# split of few queries behind at least 3072 keys, blocks of 16 to 64 tokens
+# of them, D 128 from 160), 128 (D 128 from 160); keys in sets of 128 or streams of 256, a
+# prefix split where that saves enough rounds of 256 keys, blocks of 16 to 64 tokens
 @pytest.mark.parametrize("D,Hq,Hkv,B,base,n", [
     (64, 14, 2, 16, 0, 1), (64, 14, 2, 16, 0, 96), (128, 8, 2, 16, 0, 65), (128, 8, 2, 16, 0, 9),  # 1 to 3 waves with keys
     (64, 14, 2, 16, 0, 31), (64, 14, 2, 16, 1, 33), (64, 3, 3, 32, 255, 65), (64, 5, 1, 64, 63, 129),

@@ -240,7 +240,7 @@ def test_config5_batch32_every_token_teacher_forced():
             total += len(o)
         print(f"config 5 batch 32: {total_exact} of {total} generated tokens exact; beyond-tie mismatches {worst}")
         assert not worst, worst
-        assert total_exact >= total - 2  # measured: 267 of 268 (one near-tie)
+        assert total_exact >= total - 2  # measured: 266 of 268 (two near-ties)
     finally:
         m.close()
 
