@@ -13,7 +13,7 @@
 // projection + SwiGLU; down projection + residual; then final norm + lm_head +
 // argmax.  Prompts and larger batches run RMSNorm and the fused linear layers of many rows
 // (kvc_block_qkv / swiglu / linear), with the prompts' K/V stored by the q/k/v kernel, and
-// rocBLAS with one kernel per op for the products where that is faster (fused_products).
+// rocBLAS with one kernel per op for large products of wide layers (fused_products).
 // step_path 1 runs every op as a kernel of its own; all round to fp16 at the same points.  With `graph` the
 // fused step is captured once as a HIP graph whose kernels read the step's counts
 // (rows, attention units, partial records) from device memory; each step then
@@ -209,24 +209,23 @@ struct QwenModel {
     void* vl(int l) const { return kvm.v_layer(l); }
 
     // Which products of a many-row layer run as one fused kernel (kvc_block_*) and which as
-    // rocBLAS and a kernel per op (us, op by op and fused).  Large products of wide layers
-    // belong to rocBLAS: gate|up at 1024 rows of hidden 2048 110 and 149, at 128 of 4096 72 and
-    // 56; o_proj at 1500 rows of 1536 17 and 20, at 4096 of 896 16.9 and 16.1 (few rows are level
-    // alone, but in a layer each launch saved counts: 256 rows of 4096 282 and 262 in all); q|k|v,
-    // with five more launches, later: 2048 rows of 4096 149 and 133, 3000 185 and 213.  down_proj
-    // follows its rows: up to about 1400 the fused kernel's K groups fill the chip (inter 4864,
-    // 700 rows 28.5 and 20.5; 11008, 1024 rows 111 and 86; 4864, 3000 rows 38 and 67), and a K
-    // of some 5000 is the longer chain at few rows (64 rows 11.8 and 18.6, 384 rows 33 and 20).
+    // rocBLAS and a kernel per op: fused wherever the layer is not slower for it.  Models of
+    // hidden <= 1024 are served without rocBLAS, whose loading takes a second (it had fallen into
+    // the first prompt of more than 1400 rows for a gain of 10% there): hidden 896, a layer op by
+    // op and fused at 40 rows 183 and 65 us, 700 184 and 92, 3000 279 and 246.  Wide layers fall
+    // behind with the size of gate|up, first there and at o_proj (its products alone: 512 rows of
+    // 4096 194 and 173, 700 185 and 242, 1500 335 and 473; 1500 rows of 2048 164 and 213), from
+    // some 1400 rows at down_proj (1024 rows of 4096 248 and 156, 1500 221 and 260) and, with five
+    // more launches, last at q|k|v (2048 rows of 4096 149 and 133, 3000 185 and 213).
     struct Fused { bool qkv, o, gate_up, down; };
     Fused fused_products(int M) const {
         const double H = c.hidden, QD = (double)c.n_heads * c.head_dim, KD = (double)c.n_kv_heads * c.head_dim;
-        const double I = c.inter;
         Fused f{};
         if (!block_ok) return f;
-        f.qkv = M * (QD + 2 * KD) * H <= 45e9;
-        f.o = QD <= 1024 || M <= 320 || (QD <= 2048 && M * H * QD <= 2.4e9);
-        f.gate_up = H <= 1024 || M <= 320 || M * 2 * I * H <= 16e9;
-        f.down = M <= 1400 && (I >= 6144 || (I >= 3072 && M >= 320));
+        const bool large = H > 1024 && M * 2.0 * c.inter * H > 62e9;
+        f.qkv = !large || M * (QD + 2 * KD) * H <= 45e9;
+        f.o = f.gate_up = !large;
+        f.down = !large || M <= 1400;
         return f;
     }
 
